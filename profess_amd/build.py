@@ -18,7 +18,10 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 SOURCES = ["ofd_kernels.hip", "ofd_fast.hip", "ofd_fast_d3.hip", "ofd_fast_d4.hip", "ofd_fast_f3.hip",
            "ofd_fast_f4.hip", "ofd_fast_d8.hip", "ofd_fast_f8.hip",
            "ofd_fast_d5.hip", "ofd_fast_f5.hip", "ofd_fast_d7.hip", "ofd_fast_f7.hip", "ofd_tables.hip", "ofd_plan.cpp",
-           "ofd_api.cpp", "ofd_io.cpp"]
+           "ofd_api.cpp", "ofd_io.cpp", "ofd_gen.hip"]
+# the general FP64 passes: columns by group of lengths, rows by field count and group
+SOURCES += ["ofd_gen_cols_%s.hip" % g for g in "abcde"]
+SOURCES += ["ofd_gen_rows%s_%s.hip" % (k, g) for k in "134578" for g in ("lo", "hi")]
 COMMON = ["-std=c++17", "-O3", "-fPIC", "-pthread", "-Wno-unused-result", "-Wno-unused-value"]
 DEVICE = ["--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 

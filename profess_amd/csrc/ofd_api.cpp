@@ -2831,8 +2831,9 @@ extern "C" int ofd_autotune(ofd_ctx* c, int reps, ofd_tune_result* res) {
     } else {
       // the x rows per workgroup set how the energy partials are grouped, so
       // they stay fixed: tuning never changes a result's bits
-      cy = {1, 2, 4, 8, 16};
-      cz = {1, 2, 4, 8};
+      const bool gen = !c->sp.force_generic && !fp32 && gen_path_ok(c->sp);
+      cy = gen ? std::vector<int>{8, 16, 24, 32} : std::vector<int>{1, 2, 4, 8, 16};
+      cz = gen ? cy : std::vector<int>{1, 2, 4, 8};
       cx = {0};
       cp = {1};
     }

@@ -1005,14 +1005,18 @@ __device__ __forceinline__ double epi32(const ReqDesc& D, double rho_d, double v
 // they are in flight together instead of one point at a time, and the first
 // chunk's loads are issued before the workgroup barrier that completes the
 // lines in LDS (this function starts with that barrier). The sums go to acc.
-template <int M, int KIND, int INMODE, int OUTMODE, int RPB, int NT, int LR, int PPR, typename R>
+// FM: field j of row rr sits at line j*RPB + rr instead (field-major lines).
+// OUTMODE -1: the form is the run-time `outmode`.
+template <int M, int KIND, int INMODE, int OUTMODE, int RPB, int NT, int LR, int PPR, bool FM = false, typename R>
 __device__ __forceinline__ void x_epi_points(const ReqDesc& D, const R* __restrict__ lr, long long row0,
-                                             long long nrows, int ioff, double (&acc)[kNSum]) {
+                                             long long nrows, int ioff, double (&acc)[kNSum], int outmode = OUTMODE) {
   constexpr int NF = NF_<KIND>::v;
   constexpr int EPT = (RPB * PPR + NT - 1) / NT;
   // global loads per point: u and vion, v (trial points and the optimizer
   // forms), b and w (Newton form); at most 16 doubles in flight per thread
-  constexpr int NL = 2 + (INMODE == kInPhi || OUTMODE != kOutPot ? 1 : 0) + (OUTMODE == kOutNewton ? 2 : 0);
+  constexpr int NL = 2 + (INMODE == kInPhi || OUTMODE != kOutPot ? 1 : 0) +
+                     (OUTMODE == kOutNewton || OUTMODE < 0 ? 2 : 0);
+  const int om = OUTMODE >= 0 ? OUTMODE : outmode;
   constexpr int PF = EPT < 16 / NL ? EPT : 16 / NL;
   const int nrow = (int)min((long long)RPB, nrows - row0);
   const int npts = nrow * PPR;
@@ -1021,7 +1025,7 @@ __device__ __forceinline__ void x_epi_points(const ReqDesc& D, const R* __restri
   auto gidx = [&](int e) { return PPR == 2 * M ? gbase + e : gbase + (size_t)(e / PPR) * 2 * M + e % PPR; };
   // the second vector: the phi direction of a trial point (kInPhi), the
   // search direction of the signed form, the CG direction of the Newton form
-  const bool want_v = D.v != nullptr && (INMODE == kInPhi || OUTMODE != kOutPot);
+  const bool want_v = D.v != nullptr && (INMODE == kInPhi || om != kOutPot);
 #pragma unroll
   for (int c0 = 0; c0 < EPT; c0 += PF) {
     double pu[PF], pv[PF], pion[PF], pb[PF], pw[PF];
@@ -1034,7 +1038,7 @@ __device__ __forceinline__ void x_epi_points(const ReqDesc& D, const R* __restri
       pu[q] = glb(D.u)[g];
       if (want_v) pv[q] = glb(D.v)[g];
       pion[q] = glb(D.vion)[g];
-      if (OUTMODE == kOutNewton) {
+      if (om == kOutNewton) {
         pb[q] = glb(D.bvec)[g];
         if (D.w != nullptr) pw[q] = glb(D.w)[g];
       }
@@ -1046,7 +1050,7 @@ __device__ __forceinline__ void x_epi_points(const ReqDesc& D, const R* __restri
     for (int q = 0; q < PF; ++q) {
       asm volatile("" : "+v"(pu[q]), "+v"(pion[q]));
       if (want_v) asm volatile("" : "+v"(pv[q]));
-      if (OUTMODE == kOutNewton) asm volatile("" : "+v"(pb[q]), "+v"(pw[q]));
+      if (om == kOutNewton) asm volatile("" : "+v"(pb[q]), "+v"(pw[q]));
     }
 #pragma unroll
     for (int q = 0; q < PF; ++q) {
@@ -1056,7 +1060,7 @@ __device__ __forceinline__ void x_epi_points(const ReqDesc& D, const R* __restri
       const size_t g = gidx(e);
       double o[NF];
 #pragma unroll
-      for (int j = 0; j < NF; ++j) o[j] = (double)lr[(size_t)(rr * NF + j) * LR + ii];
+      for (int j = 0; j < NF; ++j) o[j] = (double)lr[(size_t)(FM ? j * RPB + rr : rr * NF + j) * LR + ii];
       if constexpr (is_spin_kind(KIND)) {
         // both channels: the second one's inputs are loaded here
         double t1 = 0.0, t2 = 0.0, r1, r2;
@@ -1072,10 +1076,10 @@ __device__ __forceinline__ void x_epi_points(const ReqDesc& D, const R* __restri
         }
         double p1, p2;
         epi_point_spin<KIND>(D, r1, r2, pion[q], o, acc, p1, p2);
-        if (OUTMODE == kOutPot) {
+        if (om == kOutPot) {
           glb(D.out)[g] = p1;
           glb(D.out2)[g] = p2;
-        } else if (OUTMODE == kOutSigned) {
+        } else if (om == kOutSigned) {
           const double de1 = p1 * fsign(t1), de2 = p2 * fsign(t2);
           glb(D.out)[g] = de1;
           glb(D.out2)[g] = de2;
@@ -1108,9 +1112,9 @@ __device__ __forceinline__ void x_epi_points(const ReqDesc& D, const R* __restri
       double pot;
       if constexpr (sizeof(R) == 4 && (KIND == kWT3 || KIND == kWT4)) pot = epi32<KIND>(D, rho, pion[q], o, acc);
       else pot = epi<KIND>(D, rho, pion[q], o, acc);
-      if (OUTMODE == kOutPot) {
+      if (om == kOutPot) {
         glb(D.out)[g] = pot;
-      } else if (OUTMODE == kOutSigned) {
+      } else if (om == kOutSigned) {
         const double de = pot * fsign(tphi);
         glb(D.out)[g] = de;
         const double dir = D.s1 * pu[q] + (D.v != nullptr ? D.s2 * pv[q] : 0.0);

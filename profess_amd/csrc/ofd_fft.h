@@ -302,6 +302,15 @@ template <int A, int B, int S, typename C> struct BflyAB {
     }
   }
 };
+template <int S, typename C> struct Bfly<6, S, C> { __device__ static void run(C* x) { BflyAB<2, 3, S, C>::run(x); } };
+template <int S, typename C> struct Bfly<9, S, C> { __device__ static void run(C* x) { BflyAB<3, 3, S, C>::run(x); } };
+template <int S, typename C> struct Bfly<10, S, C> { __device__ static void run(C* x) { BflyAB<2, 5, S, C>::run(x); } };
+template <int S, typename C> struct Bfly<14, S, C> { __device__ static void run(C* x) { BflyAB<2, 7, S, C>::run(x); } };
+template <int S, typename C> struct Bfly<18, S, C> { __device__ static void run(C* x) { BflyAB<2, 9, S, C>::run(x); } };
+template <int S, typename C> struct Bfly<21, S, C> { __device__ static void run(C* x) { BflyAB<3, 7, S, C>::run(x); } };
+template <int S, typename C> struct Bfly<25, S, C> { __device__ static void run(C* x) { BflyAB<5, 5, S, C>::run(x); } };
+template <int S, typename C> struct Bfly<27, S, C> { __device__ static void run(C* x) { BflyAB<3, 9, S, C>::run(x); } };
+template <int S, typename C> struct Bfly<35, S, C> { __device__ static void run(C* x) { BflyAB<5, 7, S, C>::run(x); } };
 template <int S, typename C> struct Bfly<12, S, C> { __device__ static void run(C* x) { BflyAB<4, 3, S, C>::run(x); } };
 template <int S, typename C> struct Bfly<20, S, C> { __device__ static void run(C* x) { BflyAB<4, 5, S, C>::run(x); } };
 template <int S, typename C> struct Bfly<24, S, C> { __device__ static void run(C* x) { BflyAB<8, 3, S, C>::run(x); } };

@@ -150,6 +150,12 @@ int fast_eval(const ShapePlan& sp, int kind, int inmode, int outmode, int fp32, 
               hipStream_t st);
 int fast_finalize(const ShapePlan& sp, int kind, int fp32, const ReqDesc* d_descs, int nb, double* out,
                   hipStream_t st);
+// General register-resident FP64 passes for the remaining padded lengths
+// (ofd_gen.hip): the evaluation, its partials per request, plain transforms
+bool gen_path_ok(const ShapePlan& sp);
+int gen_eval(const ShapePlan& sp, int kind, int inmode, int outmode, const ReqDesc* d_descs, int nb, hipStream_t st);
+int gen_partials(const ShapePlan& sp, int kind);
+int gen_fft3d_plain(const ShapePlan& sp, int forward, const ReqDesc* d_descs, int nb, hipStream_t st);
 // Plain 3D transforms of D.u -> D.work (forward, no 1/N) or D.work -> D.out.
 int run_fft3d_plain(const ShapePlan& sp, int forward, const ReqDesc* d_descs, int nb, hipStream_t st);
 

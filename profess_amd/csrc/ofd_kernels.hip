@@ -594,9 +594,14 @@ static int eval_r(const ShapePlan& sp, int kind, int inmode, int outmode, const 
   }
 }
 
+// The general register-resident passes take the FP64 evaluations of every
+// shape whose lengths they know and the fast path does not.
+static bool use_gen(const ShapePlan& sp, int fp32) { return !sp.force_generic && !fp32 && gen_path_ok(sp); }
+
 int run_eval(const ShapePlan& sp, int kind, int inmode, int outmode, int fp32, const ReqDesc* dd, int nb,
              hipStream_t st) {
   if (!sp.force_generic && fast_path_ok(sp, kind)) return fast_eval(sp, kind, inmode, outmode, fp32, dd, nb, st);
+  if (use_gen(sp, fp32)) return gen_eval(sp, kind, inmode, outmode, dd, nb, st);
   return fp32 ? eval_r<float>(sp, kind, inmode, outmode, dd, nb, st)
               : eval_r<double>(sp, kind, inmode, outmode, dd, nb, st);
 }
@@ -605,7 +610,8 @@ int run_finalize(const ShapePlan& sp, int kind, int fp32, const ReqDesc* dd, int
   if (!sp.force_generic && fast_path_ok(sp, kind)) return fast_finalize(sp, kind, fp32, dd, nb, out, st);
   const Tiles t = tiles_for(sp, func_nf(kind), fp32 ? (int)sizeof(float2) : (int)sizeof(double2));
   (void)out;
-  hipLaunchKernelGGL(k_finalize, dim3(kNSum, nb), dim3(256), 0, st, dd, t.ntile);
+  hipLaunchKernelGGL(k_finalize, dim3(kNSum, nb), dim3(256), 0, st, dd,
+                     use_gen(sp, fp32) ? gen_partials(sp, kind) : t.ntile);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -613,6 +619,8 @@ int run_finalize(const ShapePlan& sp, int kind, int fp32, const ReqDesc* dd, int
 // Forward R2C of the real field D.u into D.work (no 1/N), backward C2R of
 // D.work into D.out (unnormalized). Used by the ion potential and forces.
 int run_fft3d_plain(const ShapePlan& sp, int forward, const ReqDesc* dd, int nb, hipStream_t st) {
+  // below 2^16 points the three launches of either form are the time
+  if (use_gen(sp, 0) && sp.d.nr >= 65536) return gen_fft3d_plain(sp, forward, dd, nb, st);
   using C = double2;
   const GridDims& d = sp.d;
   const Tiles t = tiles_for(sp, 1, (int)sizeof(C));
