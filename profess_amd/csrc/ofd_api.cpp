@@ -2817,7 +2817,7 @@ extern "C" int ofd_autotune(ofd_ctx* c, int reps, ofd_tune_result* res) {
     std::vector<double> h(n, c->num_ele / c->vol);
     HIPCHK(copy_sync(c->rho, h.data(), n * sizeof(double), hipMemcpyHostToDevice, c->st));
     graphs_clear(c->graphs);
-    const bool fast = !c->sp.force_generic && fast_path_ok(c->sp, c->kind);
+    const bool fast = !c->sp.force_generic && fast_path_ok(c->sp, c->kind, c->precision == 1);
     const int fp32 = c->precision == 1;
     std::vector<int> cy, cz, cx, cp;
     if (fast) {

@@ -41,7 +41,21 @@ __global__ void __launch_bounds__(256) k_fin(const ReqDesc* __restrict__ descs, 
 
 }  // namespace fast
 
-bool fast_path_ok(const ShapePlan& sp, int kind) { return fast_path_ok_impl(sp, kind); }
+// FP32: every shape of the line lengths below. FP64: the shapes of the
+// power-of-two plane passes (32 x 32, 64 x 64, 128 x 128), where two fused
+// passes beat the general form's three: Wang-Teter / fast against general
+// passes, 32^3 20.7 / 21.9 us, 64^3 34.5 / 35.3, 128^3 96 / 109. The general
+// passes take the rest, among them all other plane shapes (48^3 34.5 / 27.3,
+// 80^3 67.5 / 61.7, 96^3 65.2 / 64.0), two spin channels from 64^3 (59 / 53)
+// and WGC below 128^3 (32^3 31.1 / 30.1).
+bool fast_path_ok(const ShapePlan& sp, int kind, int fp32) {
+  if (!fast_path_ok_impl(sp, kind)) return false;
+  if (fp32) return true;
+  const int M = sp.d.M;
+  const bool plane = !sp.no_plane && (M == 16 || M == 32 || M == 64) && sp.d.n2 == 2 * M && !is_gp_len(sp.d.n3);
+  if (!plane) return false;
+  return kind == kWGC8 ? M == 64 : (!is_spin_kind(kind) || M == 16);
+}
 
 
 int fast_eval(const ShapePlan& sp, int kind, int inmode, int outmode, int fp32, const ReqDesc* dd, int nb,
@@ -90,10 +104,10 @@ bool fast_plane_available(const ShapePlan& sp, int kind, int fp32) {
 }
 
 // Sums the x-inverse pass's per-workgroup partials into each request's fin.
-int fast_finalize(const ShapePlan& sp, int kind, int, const ReqDesc* dd, int nb, double*, hipStream_t st) {
+int fast_finalize(const ShapePlan& sp, int kind, int fp32, const ReqDesc* dd, int nb, double*, hipStream_t st) {
   const int rpb = fast::inv_rpb(func_nf(kind), len_T(sp.d.M));
   const long long nrows = (long long)sp.d.n2 * sp.d.n3;
-  const int nwg = (int)((nrows + rpb - 1) / rpb);
+  const int nwg = gen_inverse(sp, fp32) ? gen_partials(sp, kind) : (int)((nrows + rpb - 1) / rpb);
   hipLaunchKernelGGL(fast::k_fin, dim3(kNSum, nb), dim3(256), 0, st, dd, nwg);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }

@@ -1577,6 +1577,10 @@ static inline bool is_fast_half(int m) {
 // frequency inverse)
 static inline bool is_gp_len(int n) { return n == 60 || n == 120; }
 
+// FP64 evaluations of the 128-point rows (the other plane shapes are launch
+// time) end in the general x-inverse pass: 24.8 us against 26.6 at 128^3.
+static inline bool gen_inverse(const ShapePlan& sp, int fp32) { return !fp32 && sp.d.M == 64; }
+
 inline bool fast_path_ok_impl(const ShapePlan& sp, int kind) {
   const bool xy = (is_fast_half(sp.d.M) || is_gp_len(sp.d.M)) && (is_fast_len(sp.d.n2) || is_gp_len(sp.d.n2));
   if (kind == kWGC8) return xy && is_fast_len(sp.d.n3);   // the coupled z pass has the two-stage form only
@@ -1806,10 +1810,13 @@ static int try_plane(const ShapePlan& sp, const ReqDesc* dd, int nb, hipStream_t
   if (sp.d.M == 64 && sp.d.n2 == 128) return go(integral_constant<int, 64>(), integral_constant<int, 128>());
   if (sp.d.M == 32 && sp.d.n2 == 64) return go(integral_constant<int, 32>(), integral_constant<int, 64>());
   if (sp.d.M == 16 && sp.d.n2 == 32) return go(integral_constant<int, 16>(), integral_constant<int, 32>());
+  if constexpr (sizeof(R) == 8) return 0;   // the general passes take the others in FP64
+  else {
   if (sp.d.M == 48 && sp.d.n2 == 96) return go(integral_constant<int, 48>(), integral_constant<int, 96>());
   if (sp.d.M == 40 && sp.d.n2 == 80) return go(integral_constant<int, 40>(), integral_constant<int, 80>());
   if (sp.d.M == 24 && sp.d.n2 == 48) return go(integral_constant<int, 24>(), integral_constant<int, 48>());
   return 0;
+  }
 }
 
 // Whether a plane pass (whole or split) serves this shape: the shapes
@@ -1843,7 +1850,7 @@ static void fast_chain(const ShapePlan& sp, const FastTiles& ft, const ReqDesc* 
                        const typename V2<R>::T* twx, const typename V2<R>::T* tws, const typename V2<R>::T* twy,
                        const typename V2<R>::T* twz) {
   constexpr int NF = fast::NF_<KIND>::v;
-  auto ylaunch = [&](auto sgn, hipStream_t s, int fo, int fn) {
+  [[maybe_unused]] auto ylaunch = [&](auto sgn, hipStream_t s, int fo, int fn) {
     constexpr int S = decltype(sgn)::value;
     switch (sp.d.n2) {
       case 24: launch_y<R, 24, S>(sp, ft.kby, fo, fn, dd, nb, s, twy); break;
@@ -1866,32 +1873,41 @@ static void fast_chain(const ShapePlan& sp, const FastTiles& ft, const ReqDesc* 
       case 32: launch_z<R, 32, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
       case 40: launch_z<R, 40, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
       case 48: launch_z<R, 48, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
-      case 60: launch_z<R, 60, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
+      case 60:
+        if constexpr (sizeof(R) == 4) launch_z<R, 60, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn);
+        break;
       case 64: launch_z<R, 64, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
       case 80: launch_z<R, 80, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
       case 96: launch_z<R, 96, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
-      case 120: launch_z<R, 120, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
+      case 120:
+        if constexpr (sizeof(R) == 4) launch_z<R, 120, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn);
+        break;
       case 128: launch_z<R, 128, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
       case 192: launch_z<R, 192, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
       default: launch_z<R, 256, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
     }
   };
-  const bool plane = plane_for<R>(sp);
-  if (!plane) launch_x<R, M, KIND, INMODE, OUTMODE>(sp, ft, dd, nb, st, true, twx, tws);
-  // one branch: the plane pass (or the forward y pass), z + G-space, inverse y
-  auto branch = [&](hipStream_t s, int fo, int fn) {
+  if constexpr (sizeof(R) == 8) {
+    // the plane shapes only (fast_path_ok)
+    const int pl = try_plane<R, KIND, INMODE>(sp, dd, nb, st, twx, tws, twy, 0, NF);
+    zlaunch(st, pl > 1 ? pl : 1, 0, NF);
+    launch_y<R, 2 * M, +1>(sp, ft.kby, 0, NF, dd, nb, st, twy);
+    if (gen_inverse(sp, 0)) gen_rows_inv(sp, KIND, INMODE, OUTMODE, dd, nb, st);
+    else if constexpr (M < 64) launch_x<R, M, KIND, INMODE, OUTMODE>(sp, ft, dd, nb, st, false, twx, tws);
+  } else {
+    const bool plane = plane_for<R>(sp);
+    if (!plane) launch_x<R, M, KIND, INMODE, OUTMODE>(sp, ft, dd, nb, st, true, twx, tws);
     int sy = 1;
     if (plane) {
-      const int pl = try_plane<R, KIND, INMODE>(sp, dd, nb, s, twx, tws, twy, fo, fn);
+      const int pl = try_plane<R, KIND, INMODE>(sp, dd, nb, st, twx, tws, twy, 0, NF);
       sy = pl > 1 ? pl : 1;   // row classes the z pass joins
     } else {
-      ylaunch(std::integral_constant<int, -1>(), s, fo, fn);
+      ylaunch(std::integral_constant<int, -1>(), st, 0, NF);
     }
-    zlaunch(s, sy, fo, fn);
-    ylaunch(std::integral_constant<int, +1>(), s, fo, fn);
-  };
-  branch(st, 0, NF);
-  launch_x<R, M, KIND, INMODE, OUTMODE>(sp, ft, dd, nb, st, false, twx, tws);
+    zlaunch(st, sy, 0, NF);
+    ylaunch(std::integral_constant<int, +1>(), st, 0, NF);
+    launch_x<R, M, KIND, INMODE, OUTMODE>(sp, ft, dd, nb, st, false, twx, tws);
+  }
 }
 
 template <typename R, int KIND, int INMODE, int OUTMODE>
@@ -1905,18 +1921,26 @@ static int fast_eval_t(const ShapePlan& sp, const ReqDesc* dd, int nb, hipStream
     twx = sp.tw_x; tws = sp.tw_s; twy = sp.tw_y; twz = sp.tw_z;
   }
   (void)f32;
-  switch (sp.d.M) {
-    case 16: fast_chain<R, KIND, INMODE, OUTMODE, 16>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-    case 24: fast_chain<R, KIND, INMODE, OUTMODE, 24>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-    case 32: fast_chain<R, KIND, INMODE, OUTMODE, 32>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-    case 40: fast_chain<R, KIND, INMODE, OUTMODE, 40>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-    case 48: fast_chain<R, KIND, INMODE, OUTMODE, 48>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-    case 60: fast_chain<R, KIND, INMODE, OUTMODE, 60>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-    case 96: fast_chain<R, KIND, INMODE, OUTMODE, 96>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-    case 120: fast_chain<R, KIND, INMODE, OUTMODE, 120>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-    case 64: fast_chain<R, KIND, INMODE, OUTMODE, 64>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-    case 128: fast_chain<R, KIND, INMODE, OUTMODE, 128>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-    default: fast_chain<R, KIND, INMODE, OUTMODE, 256>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+  if constexpr (sizeof(R) == 8) {   // the plane shapes
+    switch (sp.d.M) {
+      case 16: fast_chain<R, KIND, INMODE, OUTMODE, 16>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 32: fast_chain<R, KIND, INMODE, OUTMODE, 32>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      default: fast_chain<R, KIND, INMODE, OUTMODE, 64>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+    }
+  } else {
+    switch (sp.d.M) {
+      case 16: fast_chain<R, KIND, INMODE, OUTMODE, 16>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 24: fast_chain<R, KIND, INMODE, OUTMODE, 24>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 32: fast_chain<R, KIND, INMODE, OUTMODE, 32>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 40: fast_chain<R, KIND, INMODE, OUTMODE, 40>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 48: fast_chain<R, KIND, INMODE, OUTMODE, 48>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 60: fast_chain<R, KIND, INMODE, OUTMODE, 60>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 96: fast_chain<R, KIND, INMODE, OUTMODE, 96>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 120: fast_chain<R, KIND, INMODE, OUTMODE, 120>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 64: fast_chain<R, KIND, INMODE, OUTMODE, 64>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 128: fast_chain<R, KIND, INMODE, OUTMODE, 128>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      default: fast_chain<R, KIND, INMODE, OUTMODE, 256>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+    }
   }
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }

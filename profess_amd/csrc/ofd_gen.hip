@@ -35,7 +35,7 @@ static RowsFn rows_of(int kind, int m) {
 static int rpb_of(int kind, int m) {
   switch (m) {
 #define X(N, A, B, T_) \
-  case N: return row_rpb(N, kind == kPlain ? 1 : func_nf(kind), T_, L<N>::LINE);
+  case N: return row_rpb(N, kind == kPlain ? 1 : func_nf(kind), T_, InvLine<N>::BYTES);
     OFD_GEN_ROWS(X)
 #undef X
     default: return 1;
@@ -66,6 +66,11 @@ int gen_eval(const ShapePlan& sp, int kind, int inmode, int outmode, const ReqDe
   cz.z(kind, dd, d, nb, sp.kb_z, sp.tw_z, st);
   cy.cols(+1, dd, d.nc, y_cols(d), nf, nb, sp.kb_y, sp.tw_y, st);
   rows(false, inmode, outmode, dd, d, nb, sp.tw_x, sp.tw_s, st);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+int gen_rows_inv(const ShapePlan& sp, int kind, int inmode, int outmode, const ReqDesc* dd, int nb, hipStream_t st) {
+  gen::rows_of(kind, sp.d.M)(false, inmode, outmode, dd, sp.d, nb, sp.tw_x, sp.tw_s, st);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

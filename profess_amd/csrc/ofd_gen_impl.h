@@ -1,6 +1,6 @@
 // Register-resident two-stage FFT passes in FP64 for every grid length that
 // PadFFTdims can pad to: the products of 2, 3, 5 and 7 from 16 to 256 along y
-// and z, and n1/2 from 9 to 128 along x (SetupFFT.f90:275-380). Rows of 16
+// and z, and n1/2 from 9 to 128, and 256, along x (SetupFFT.f90:275-380). Rows of 16
 // points stay on the staged passes, which serve the 16^3 grids of the
 // reference's sample runs: the solves compared with those runs follow
 // recurrences of some 200 steps that carry a last-bit difference along, and
@@ -54,7 +54,7 @@ constexpr int kPlain = 9;   // one real field, no functional (per-geometry table
   X(256, 16, 16, 16)
 #define OFD_GEN_COLS(X) OFD_GEN_A(X) OFD_GEN_B(X) OFD_GEN_C(X) OFD_GEN_D(X) OFD_GEN_E(X)
 #define OFD_GEN_ROWS_LO(X) OFD_GEN_SHORT(X) OFD_GEN_A(X)
-#define OFD_GEN_ROWS_HI(X) OFD_GEN_B(X) OFD_GEN_C(X)
+#define OFD_GEN_ROWS_HI(X) OFD_GEN_B(X) OFD_GEN_C(X) X(256, 16, 16, 16)
 #define OFD_GEN_ROWS(X) OFD_GEN_ROWS_LO(X) OFD_GEN_ROWS_HI(X)
 
 template <int N> struct Split;
@@ -246,6 +246,16 @@ __device__ __forceinline__ void inv_s(double2 (&xs)[L<N>::NS], double2 (&xc)[L<N
   __syncthreads();
 }
 
+// The twiddle pointer, hidden from the optimizer and tied to a thread's last
+// result so far: the loads of the transform that follows are issued after it.
+// Left alone they are hoisted over the G-space operator, up to 4 (R2 - 1)
+// more VGPRs alive with the line's data (k_zgop<128>: 218 VGPRs, two waves per
+// SIMD).
+__device__ __forceinline__ const double2* again(const double2* p, double done) {
+  asm volatile("" : "+s"(p) : "v"(done));
+  return p;
+}
+
 // ------------------------------------------------------------ columns
 // A set of equal columns of one field: column e starts at
 // (e / inner) * outer + e % inner and its points are `es` apart. y: inner =
@@ -254,6 +264,27 @@ struct Cols {
   unsigned ncol, inner, outer, es;
 };
 
+// Element access by 32-bit byte offset from a workgroup-uniform base (a
+// field's bytes stay below 2^28 at the lengths served here): scalar base and
+// one offset register per element. offs() hides an offset from the optimizer
+// where a kernel uses it again, so that the elements' offsets are formed anew
+// (one add each) instead of staying alive through the transforms.
+__device__ __forceinline__ double2 ld16(gptr<const double2> b, unsigned off) {
+  return ldc((gptr<const double2>)((gptr<const char>)b + off));
+}
+__device__ __forceinline__ double ld8(gptr<const double> b, unsigned off) {
+  return *(gptr<const double>)((gptr<const char>)b + off);
+}
+__device__ __forceinline__ void st16(gptr<double2> b, unsigned off, const double2& v) {
+  stc((gptr<double2>)((gptr<char>)b + off), v);
+}
+__device__ __forceinline__ unsigned offs(unsigned o) {
+  asm volatile("" : "+v"(o));
+  return o;
+}
+
+// Elements c + R2 m of a thread's stage-1 columns, or k1 + R1 k2 of its
+// stage-2 rows; o: byte offset of the line, es: bytes between its points.
 template <int N> __device__ __forceinline__ void load_cols(double2 (&xc)[L<N>::NC], gptr<const double2> b, unsigned o,
                                                            unsigned es, int t) {
   using G = L<N>;
@@ -261,7 +292,7 @@ template <int N> __device__ __forceinline__ void load_cols(double2 (&xc)[L<N>::N
   for (int j = 0; j < G::J1; ++j)
     if (G::col_ok(t, j)) {
 #pragma unroll
-      for (int m = 0; m < G::R1; ++m) xc[j * G::R1 + m] = ldc(b + (o + (unsigned)(t + G::T * j + G::R2 * m) * es));
+      for (int m = 0; m < G::R1; ++m) xc[j * G::R1 + m] = ld16(b, o + (unsigned)t * es + (unsigned)(G::T * j + G::R2 * m) * es);
     }
 }
 template <int N> __device__ __forceinline__ void store_cols(const double2 (&xc)[L<N>::NC], gptr<double2> b, unsigned o,
@@ -271,7 +302,7 @@ template <int N> __device__ __forceinline__ void store_cols(const double2 (&xc)[
   for (int j = 0; j < G::J1; ++j)
     if (G::col_ok(t, j)) {
 #pragma unroll
-      for (int m = 0; m < G::R1; ++m) stc(b + (o + (unsigned)(t + G::T * j + G::R2 * m) * es), xc[j * G::R1 + m]);
+      for (int m = 0; m < G::R1; ++m) st16(b, o + (unsigned)t * es + (unsigned)(G::T * j + G::R2 * m) * es, xc[j * G::R1 + m]);
     }
 }
 template <int N> __device__ __forceinline__ void load_rows(double2 (&xs)[L<N>::NS], gptr<const double2> b, unsigned o,
@@ -281,7 +312,7 @@ template <int N> __device__ __forceinline__ void load_rows(double2 (&xs)[L<N>::N
   for (int q = 0; q < G::J2; ++q)
     if (G::row_ok(t, q)) {
 #pragma unroll
-      for (int k = 0; k < G::R2; ++k) xs[q * G::R2 + k] = ldc(b + (o + (unsigned)(t + G::T * q + G::R1 * k) * es));
+      for (int k = 0; k < G::R2; ++k) xs[q * G::R2 + k] = ld16(b, o + (unsigned)t * es + (unsigned)(G::T * q + G::R1 * k) * es);
     }
 }
 template <int N> __device__ __forceinline__ void store_rows(const double2 (&xs)[L<N>::NS], gptr<double2> b, unsigned o,
@@ -291,13 +322,11 @@ template <int N> __device__ __forceinline__ void store_rows(const double2 (&xs)[
   for (int q = 0; q < G::J2; ++q)
     if (G::row_ok(t, q)) {
 #pragma unroll
-      for (int k = 0; k < G::R2; ++k) stc(b + (o + (unsigned)(t + G::T * q + G::R1 * k) * es), xs[q * G::R2 + k]);
+      for (int k = 0; k < G::R2; ++k) st16(b, o + (unsigned)t * es + (unsigned)(G::T * q + G::R1 * k) * es, xs[q * G::R2 + k]);
     }
 }
 
-// In-place transform of the columns of field blockIdx.y. Element offsets are
-// 32-bit from the field's uniform base (a field has K1 n2 n3 < 2^24 elements
-// at the lengths served here).
+// In-place transform of the columns of field blockIdx.y.
 template <int N, int S>
 __global__ void __launch_bounds__(256) k_cols(const ReqDesc* __restrict__ descs, long long nc, Cols cs,
                                               const double2* __restrict__ tw, int kb) {
@@ -308,18 +337,18 @@ __global__ void __launch_bounds__(256) k_cols(const ReqDesc* __restrict__ descs,
   const unsigned col = (unsigned)xcd_block(blockIdx.x, gridDim.x) * kb + c;
   const bool active = t < G::T && col < cs.ncol;
   const unsigned grp = active ? col / cs.inner : 0;
-  const unsigned o = active ? grp * cs.outer + (col - grp * cs.inner) : 0;
+  const unsigned o = active ? (grp * cs.outer + (col - grp * cs.inner)) * 16u : 0, es = cs.es * 16u;
   gptr<double2> base = glb(reinterpret_cast<double2*>(D.work)) + (size_t)blockIdx.y * nc;
   double* line = reinterpret_cast<double*>(smem) + (size_t)c * G::LINE;
   double2 xc[G::NC], xs[G::NS];
   if constexpr (S < 0) {
-    if (active) load_cols<N>(xc, base, o, cs.es, t);
+    if (active) load_cols<N>(xc, base, o, es, t);
     fwd_s<N>(xc, xs, line, t, tw, active);
-    if (active) store_rows<N>(xs, base, o, cs.es, t);
+    if (active) store_rows<N>(xs, base, o, es, t);
   } else {
-    if (active) load_rows<N>(xs, base, o, cs.es, t);
+    if (active) load_rows<N>(xs, base, o, es, t);
     inv_s<N>(xs, xc, line, t, tw, active);
-    if (active) store_cols<N>(xc, base, o, cs.es, t);
+    if (active) store_cols<N>(xc, base, o, es, t);
   }
 }
 
@@ -356,18 +385,21 @@ __global__ void __launch_bounds__(256) k_zgop(const ReqDesc* __restrict__ descs,
   const double invn = 1.0 / (double)d.nr;
   gptr<double2> base = glb(reinterpret_cast<double2*>(D.work)) + (size_t)f * d.nc;
   double* line = reinterpret_cast<double*>(smem) + (size_t)c * G::LINE;
-  double2 xc[G::NC], xs[G::NS];
-  if (active) load_cols<N>(xc, base, col, es, t);
+  // the inverse writes an array of its own: lanes that skip the branches would
+  // keep xc's old contents alive through the whole pass otherwise
+  double2 xc[G::NC], xs[G::NS], yc[G::NC];
+  if (active) load_cols<N>(xc, base, col * 16u, es * 16u, t);
   fwd_s<N>(xc, xs, line, t, tw, active);
   if (active) {
     if (f != 0 && f < fvw) {
       gptr<const double> wk = glb(D.wtk);
+      const unsigned ow = (col + (unsigned)t * es) * 8u;
 #pragma unroll
       for (int q = 0; q < G::J2; ++q)
         if (G::row_ok(t, q)) {
 #pragma unroll
           for (int k = 0; k < G::R2; ++k) {
-            const double s = wk[col + (unsigned)(t + G::T * q + G::R1 * k) * es];
+            const double s = ld8(wk, ow + (unsigned)(G::T * q + G::R1 * k) * (es * 8u));
             xs[q * G::R2 + k].x *= s;
             xs[q * G::R2 + k].y *= s;
           }
@@ -389,8 +421,8 @@ __global__ void __launch_bounds__(256) k_zgop(const ReqDesc* __restrict__ descs,
         }
     }
   }
-  inv_s<N>(xs, xc, line, t, tw, active);
-  if (active) store_cols<N>(xc, base, col, es, t);
+  inv_s<N>(xs, yc, line, t, again(tw, xs[G::NS - 1].y), active);
+  if (active) store_cols<N>(yc, base, offs(col * 16u), es * 16u, t);
 }
 
 // z columns of the WGC fields with the coupled operator, as fast::k_fz_wgc:
@@ -412,14 +444,16 @@ __global__ void __launch_bounds__(256) k_zwgc(const ReqDesc* __restrict__ descs,
   const double invn = 1.0 / (double)d.nr;
   gptr<double2> base = glb(reinterpret_cast<double2*>(D.work)) + (size_t)f0 * d.nc;
   double* line = reinterpret_cast<double*>(smem) + (size_t)c * G::LINE;
-  double2 xc[G::NC], xs[G::NS], xa[G::NS];
-  auto get = [&](int j) {
-    if (active) load_cols<N>(xc, base + (size_t)j * d.nc, col, es, t);
-    fwd_s<N>(xc, xs, line, t, tw, active);
+  // every transform between arrays of its own (see k_zgop)
+  auto get = [&](int j, double2 (&xs)[G::NS]) {
+    double2 xc[G::NC];
+    if (active) load_cols<N>(xc, base + (size_t)j * d.nc, offs(col * 16u), es * 16u, t);
+    fwd_s<N>(xc, xs, line, t, again(tw, xc[G::NC - 1].y), active);
   };
-  auto put = [&](int j) {
-    inv_s<N>(xs, xc, line, t, tw, active);
-    if (active) store_cols<N>(xc, base + (size_t)j * d.nc, col, es, t);
+  auto put = [&](int j, double2 (&xs)[G::NS]) {
+    double2 xc[G::NC];
+    inv_s<N>(xs, xc, line, t, again(tw, xs[G::NS - 1].y), active);
+    if (active) store_cols<N>(xc, base + (size_t)j * d.nc, offs(col * 16u), es * 16u, t);
   };
   // each(fn): fn(slot, i3) for every point the thread holds
   auto each = [&](auto&& fn) {
@@ -435,99 +469,144 @@ __global__ void __launch_bounds__(256) k_zwgc(const ReqDesc* __restrict__ descs,
     const int i2 = active ? (int)(col / d.K1) : 0, m1 = active ? (int)col - i2 * d.K1 : 0;
     const G2Col g2(D, m1, i2 > d.n2 / 2 ? i2 - d.n2 : i2);
     for (int j = 0; j < 2; ++j) {
-      get(j);
+      double2 xs[G::NS];
+      get(j, xs);
       each([&](int s, int i3) {
         const double q2 = g2.at(i3 > N / 2 ? i3 - N : i3);
         const double sc = j == 0 ? (q2 > 0.0 ? 4.0 * kPi / q2 * invn : 0.0) : q2 * invn;
         xs[s].x *= sc;
         xs[s].y *= sc;
       });
-      put(j);
+      put(j, xs);
     }
     return;
   }
   gptr<const double> wk = glb(D.wgck);
-  get(0);
+  double2 xa[G::NS], xb[G::NS];
+  get(0, xa);
+  {
+    double2 xs[G::NS];
+    each([&](int s, int i3) {
+      const double k3 = ld8(wk + 2 * d.nc, (col + (unsigned)i3 * es) * 8u) * invn;
+      xs[s].x = k3 * xa[s].x;
+      xs[s].y = k3 * xa[s].y;
+    });
+    put(0, xs);
+  }
+  {
+    double2 xs[G::NS];
+    get(1, xs);
+    each([&](int s, int i3) {
+      const unsigned gi = (col + (unsigned)i3 * es) * 8u;
+      const double k1 = ld8(wk, gi) * invn, k2 = ld8(wk + d.nc, gi) * invn, k4 = ld8(wk + 3 * d.nc, gi) * invn;
+      const double2 a = xa[s], b = xs[s];
+      xb[s].x = k1 * a.x + k2 * b.x;
+      xb[s].y = k1 * a.y + k2 * b.y;
+      xs[s].x = k2 * a.x + k4 * b.x;
+      xs[s].y = k2 * a.y + k4 * b.y;
+    });
+    put(1, xs);
+  }
+  double2 xs[G::NS];
+  get(2, xs);
   each([&](int s, int i3) {
-    const double k3 = wk[2 * d.nc + (col + (unsigned)i3 * es)] * invn;
-    xa[s] = xs[s];
-    xs[s].x *= k3;
-    xs[s].y *= k3;
+    const double k3 = ld8(wk + 2 * d.nc, (col + (unsigned)i3 * es) * 8u) * invn;
+    xs[s].x = xb[s].x + k3 * xs[s].x;
+    xs[s].y = xb[s].y + k3 * xs[s].y;
   });
-  put(0);
-  get(1);
-  each([&](int s, int i3) {
-    const unsigned gi = col + (unsigned)i3 * es;
-    const double k1 = wk[gi] * invn, k2 = wk[d.nc + gi] * invn, k4 = wk[3 * d.nc + gi] * invn;
-    const double2 a = xa[s], b = xs[s];
-    xa[s].x = k1 * a.x + k2 * b.x;
-    xa[s].y = k1 * a.y + k2 * b.y;
-    xs[s].x = k2 * a.x + k4 * b.x;
-    xs[s].y = k2 * a.y + k4 * b.y;
-  });
-  put(1);
-  get(2);
-  each([&](int s, int i3) {
-    const double k3 = wk[2 * d.nc + (col + (unsigned)i3 * es)] * invn;
-    xs[s].x = xa[s].x + k3 * xs[s].x;
-    xs[s].y = xa[s].y + k3 * xs[s].y;
-  });
-  put(2);
+  put(2, xs);
 }
 
 // ------------------------------------------------------------ x rows
 template <int KIND> struct NFg { static constexpr int v = fast::NF_<KIND>::v; };
 template <> struct NFg<kPlain> { static constexpr int v = 1; };
 
-// Rows per workgroup: whole rows of NF lines, at most 256 threads (64 for the
-// short rows of small grids, which have few workgroups to fill the chip with)
-// and 48 KB of complex lines, the count that leaves the fewest lanes idle.
-constexpr int row_rpb(int m, int nf, int t, int line) {
-  const int cap = m <= 24 ? 64 : (m <= 48 ? 128 : 256);
+// Rows per workgroup: whole rows of NF lines, at most 48 KB of lines (`bytes`
+// each), the count that leaves the fewest lanes idle within 128 threads (64 for
+// the short rows of small grids, which have few workgroups to fill the chip
+// with), or within 256 where 128 would leave one lane in eight idle. (256
+// throughout: 200^3 WT inverse 92 against 83 us, 100^3 15.8 against 14.2.)
+constexpr int row_rpb(int m, int nf, int t, int bytes) {
   int best = 1;
   double eff = 0.0;
-  for (int r = 1; r * nf * t <= (cap > nf * t ? cap : nf * t); ++r) {
-    if (r > 1 && (long long)r * nf * line * 16 > 49152) break;
-    const int th = r * nf * t, up = (th + 63) / 64 * 64;
-    const double e = (double)th / up;
-    if (e >= eff) {
-      eff = e;
-      best = r;
+  for (int cap = m <= 24 ? 64 : 128; cap <= 256 && eff < 0.875; cap *= 2)
+    for (int r = 1; r == 1 || r * nf * t <= cap; ++r) {
+      if (r > 1 && (long long)r * nf * bytes > 49152) break;
+      const int th = r * nf * t, up = (th + 63) / 64 * 64;
+      const double e = (double)th / up;
+      if (e >= eff) {
+        eff = e;
+        best = r;
+      }
     }
-  }
   return best;
 }
+// The inverse pass. Rows with 15 points and more per thread (60, 112, 120, 128)
+// exchange one real component at a time and run their epilogue over the two
+// halves of each row in turn (columns m < R1/2 of every thread are the row's
+// first M reals): at 16 points a thread complex lines leave 9 waves per CU
+// (256^3 WT 221 -> 200 us for the pass, 120^3 30.7 -> 28.0). With fewer points
+// a thread the complex lines are faster (180^3 58.8 against 67.5 us).
+template <int M> struct InvLine {
+  static constexpr bool SC = L<M>::R1 % 2 == 0 && std::max(L<M>::NC, L<M>::NS) >= 15;
+  static constexpr int LINE = L<M>::LINE;   // reals (SC) or complex
+  static constexpr int BYTES = LINE * (SC ? 8 : 16);
+};
 template <int M, int KIND> struct RowGeo {
-  static constexpr int NF = NFg<KIND>::v, T = L<M>::T, LINE = L<M>::LINE;
-  static constexpr int RPB = row_rpb(M, NF, T, LINE);
+  static constexpr int NF = NFg<KIND>::v, T = L<M>::T;
+  static constexpr int RPB = row_rpb(M, NF, T, InvLine<M>::BYTES);
   static constexpr int NL = RPB * NF;                          // lines per workgroup, field-major
   static constexpr int NT = (NL * T + 63) / 64 * 64;           // threads
-  static constexpr size_t LDS = (size_t)NL * LINE * sizeof(double2);
+  static constexpr size_t LDS = (size_t)NL * InvLine<M>::BYTES;
+};
+// The forward pass: one wave per field with as many rows as it has lanes for,
+// so that no wave forms two kinds of field (a divergent wave pays for each);
+// the short rows of small grids pack their lines densely instead, for more
+// workgroups. Rows of 60 points and more (WGC 36) exchange one real component
+// at a time (half the LDS, twice the waves per CU: 256^3 WT 294 -> 212 us for
+// the pass, 200^3 89 -> 75, 108^3 WGC 36.4 -> 32.0); below that the complex
+// exchange is 5 % faster.
+template <int M, int KIND> struct RowGeoF {
+  static constexpr int NF = NFg<KIND>::v, T = L<M>::T, LINE = L<M>::LINE;
+  static constexpr bool SC = M >= (KIND == kWGC8 ? 36 : 60), WF = M > 24;
+  static constexpr int RPB = WF ? 64 / T : row_rpb(M, NF, T, 16 * LINE);
+  static constexpr int NL = RPB * NF;
+  static constexpr int NT = WF ? NF * 64 : (NL * T + 63) / 64 * 64;
+  static constexpr size_t LDS = std::max((size_t)NL * LINE * (SC ? 1 : 2), KIND == kWGC8 ? (size_t)RPB * 4 * M : (size_t)0) *
+                                sizeof(double);   // the lines; before them WGC's two powers of each point
 };
 
 // Rows along x, forward: every line forms its field from rho, transforms it
 // and leaves it in LDS; then the workgroup's threads write the R2C split of
 // all lines, consecutive threads on consecutive k (whole cache lines, where a
-// line's own T threads would write T elements at a time). Lines are ordered
-// field by field, so a wave mostly forms one kind of field.
+// line's own T threads would write T elements at a time).
 template <int M, int KIND>
-__global__ void __launch_bounds__(256) k_rows_fwd(const ReqDesc* __restrict__ descs, GridDims d,
+__global__ void __launch_bounds__((RowGeoF<M, KIND>::NT)) k_rows_fwd(const ReqDesc* __restrict__ descs, GridDims d,
                                                   const double2* __restrict__ tw, const double2* __restrict__ tws,
                                                   int inmode) {
   using G = L<M>;
-  using W = RowGeo<M, KIND>;
+  using W = RowGeoF<M, KIND>;
   extern __shared__ __align__(16) unsigned char smem[];
-  double2* lds = reinterpret_cast<double2*>(smem);
+  double* lds = reinterpret_cast<double*>(smem);
   const ReqDesc& D = descs[blockIdx.y];
-  const int line = threadIdx.x / G::T, t = threadIdx.x % G::T;
-  const int f = line / W::RPB, r = line - f * W::RPB;
+  const int lane = W::WF ? threadIdx.x % 64 : threadIdx.x;
+  const int t = lane % G::T;
+  int f, r;
+  if constexpr (W::WF) {
+    f = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    r = lane / G::T;
+  } else {
+    f = lane / G::T / W::RPB;
+    r = lane / G::T - f * W::RPB;
+  }
+  const int line = f * W::RPB + r;
   const long long nrows = (long long)d.n2 * d.n3;
   const long long row0 = (long long)xcd_block(blockIdx.x, gridDim.x) * W::RPB;
-  const bool active = line < W::NL && row0 + r < nrows;
+  const bool active = f < W::NF && r < W::RPB && row0 + r < nrows;
   double2 xc[G::NC], xs[G::NS];
   if constexpr (KIND == kWGC8) {
     // each point's two powers once per row, shared through LDS
-    double* pw = reinterpret_cast<double*>(smem);
+    double* pw = lds;
     const int nrow = (int)min((long long)W::RPB, nrows - row0);
     for (int e = threadIdx.x; e < nrow * 2 * M; e += W::NT) {
       const size_t g = (size_t)row0 * (2 * M) + e;
@@ -587,34 +666,85 @@ __global__ void __launch_bounds__(256) k_rows_fwd(const ReqDesc* __restrict__ de
       }
     }
   }
-  double2* mine = lds + (size_t)line * G::LINE;
-  fwd_c<M>(xc, xs, mine, t, tw, active);
-  if (active) {
-#pragma unroll
-    for (int q = 0; q < G::J2; ++q)
-      if (G::row_ok(t, q)) {
-#pragma unroll
-        for (int k2 = 0; k2 < G::R2; ++k2) mine[t + G::T * q + G::R1 * k2] = xs[q * G::R2 + k2];
-      }
-  }
-  __syncthreads();
-  const int nrow = (int)min((long long)W::RPB, nrows - row0);
+  // The split X[k] = E[k] + W^k O[k] of Z reads Z[k] and Z[M-k]; an element's
+  // place and factor are the same for every field.
+  constexpr int PER = (W::RPB * (M + 1) + W::NT - 1) / W::NT;
+  const int nel = (int)min((long long)W::RPB, nrows - row0) * (M + 1);
   gptr<double2> work = glb(reinterpret_cast<double2*>(D.work));
-  // field by field: the workgroup's rows of a field are contiguous in memory
+  auto natural = [&](auto* mine, auto&& part) {
+    if (active) {
 #pragma unroll
-  for (int ff = 0; ff < W::NF; ++ff) {
-    gptr<double2> out = work + (size_t)ff * d.nc + (size_t)row0 * (M + 1);
-    for (int e = threadIdx.x; e < nrow * (M + 1); e += W::NT) {
+      for (int q = 0; q < G::J2; ++q)
+        if (G::row_ok(t, q)) {
+#pragma unroll
+          for (int k2 = 0; k2 < G::R2; ++k2) mine[t + G::T * q + G::R1 * k2] = part(xs[q * G::R2 + k2]);
+        }
+    }
+    __syncthreads();
+  };
+  if constexpr (W::SC) {
+    // real parts through LDS first (giving Re E and Im O), then the imaginary parts
+    double* mine = lds + (size_t)line * G::LINE;
+    fwd_s<M>(xc, xs, mine, t, tw, active);
+    double er[PER][W::NF], oi[PER][W::NF];
+    natural(mine, [](const double2& z) { return z.x; });
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const int e = min((int)threadIdx.x + q * W::NT, nel - 1);
       const int rr = e / (M + 1), k = e - rr * (M + 1);
-      const double2* z = lds + (size_t)(ff * W::RPB + rr) * G::LINE;
-      const double2 zk = z[k == M ? 0 : k], zm = z[k == 0 ? 0 : M - k];
-      const double er = 0.5 * (zk.x + zm.x), ei = 0.5 * (zk.y - zm.y);
-      const double orr = 0.5 * (zk.y + zm.y), oi = -0.5 * (zk.x - zm.x);
+      const double* z = lds + (size_t)rr * G::LINE;
+#pragma unroll
+      for (int ff = 0; ff < W::NF; ++ff) {
+        const double zk = z[ff * W::RPB * G::LINE + (k == M ? 0 : k)],
+                     zm = z[ff * W::RPB * G::LINE + (k == 0 ? 0 : M - k)];
+        er[q][ff] = 0.5 * (zk + zm);
+        oi[q][ff] = -0.5 * (zk - zm);
+      }
+    }
+    __syncthreads();
+    natural(mine, [](const double2& z) { return z.y; });
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const int e = threadIdx.x + q * W::NT;
+      if (e >= nel) break;
+      const int rr = e / (M + 1), k = e - rr * (M + 1);
       const double2 w = tws[k];
-      double2 x;
-      x.x = er + (w.x * orr - w.y * oi);
-      x.y = ei + (w.x * oi + w.y * orr);
-      stc(out + e, x);
+      const double* z = lds + (size_t)rr * G::LINE;
+      gptr<double2> out = work + ((size_t)row0 * (M + 1) + e);
+#pragma unroll
+      for (int ff = 0; ff < W::NF; ++ff) {
+        const double zk = z[ff * W::RPB * G::LINE + (k == M ? 0 : k)],
+                     zm = z[ff * W::RPB * G::LINE + (k == 0 ? 0 : M - k)];
+        const double ei = 0.5 * (zk - zm), orr = 0.5 * (zk + zm);
+        double2 x;
+        x.x = er[q][ff] + (w.x * orr - w.y * oi[q][ff]);
+        x.y = ei + (w.x * oi[q][ff] + w.y * orr);
+        stc(out + (size_t)ff * d.nc, x);
+      }
+    }
+  } else {
+    double2* all = reinterpret_cast<double2*>(smem);
+    double2* mine = all + (size_t)line * G::LINE;
+    fwd_c<M>(xc, xs, mine, t, tw, active);
+    natural(mine, [](const double2& z) { return z; });
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const int e = threadIdx.x + q * W::NT;
+      if (e >= nel) break;
+      const int rr = e / (M + 1), k = e - rr * (M + 1);
+      const double2 w = tws[k];
+      const double2* z = all + (size_t)rr * G::LINE;
+      gptr<double2> out = work + ((size_t)row0 * (M + 1) + e);
+#pragma unroll
+      for (int ff = 0; ff < W::NF; ++ff) {
+        const double2 zk = z[ff * W::RPB * G::LINE + (k == M ? 0 : k)], zm = z[ff * W::RPB * G::LINE + (k == 0 ? 0 : M - k)];
+        const double er = 0.5 * (zk.x + zm.x), ei = 0.5 * (zk.y - zm.y);
+        const double orr = 0.5 * (zk.y + zm.y), oi = -0.5 * (zk.x - zm.x);
+        double2 x;
+        x.x = er + (w.x * orr - w.y * oi);
+        x.y = ei + (w.x * oi + w.y * orr);
+        stc(out + (size_t)ff * d.nc, x);
+      }
     }
   }
 }
@@ -629,8 +759,8 @@ __global__ void __launch_bounds__(256) k_rows_inv(const ReqDesc* __restrict__ de
                                                   int outmode) {
   using G = L<M>;
   using W = RowGeo<M, KIND>;
+  using Q = InvLine<M>;
   extern __shared__ __align__(16) unsigned char smem[];
-  double2* lds = reinterpret_cast<double2*>(smem);
   const ReqDesc& D = descs[blockIdx.y];
   const int line = threadIdx.x / G::T, t = threadIdx.x % G::T;
   const int f = line / W::RPB, r = line - f * W::RPB;
@@ -651,60 +781,118 @@ __global__ void __launch_bounds__(256) k_rows_inv(const ReqDesc* __restrict__ de
 #pragma unroll
     for (int q = 0; q < PER; ++q) v[ff][q] = ldc(in + min((int)threadIdx.x + q * W::NT, nel - 1));
   }
-#pragma unroll
-  for (int q = 0; q < PER; ++q) {
-    const int e = threadIdx.x + q * W::NT;
-    if (e < nel) {
-      const int rr = e / (M + 1), k = e - rr * (M + 1);
-#pragma unroll
-      for (int ff = 0; ff < W::NF; ++ff) lds[(size_t)(ff * W::RPB + rr) * G::LINE + k] = v[ff][q];
-    }
-  }
-  __syncthreads();
-  double2* mine = lds + (size_t)line * G::LINE;
+  // merge of X[k] and X[M-k] (C2R; the imaginary parts of X[0] and X[M] drop)
+  auto merge = [&](int k, double er, double dr, double ei, double di) {
+    const double2 w = tws[k];
+    const double orr = w.x * dr + w.y * di, oi = w.x * di - w.y * dr;
+    return make_double2(er - oi, ei + orr);
+  };
   double2 xc[G::NC], xs[G::NS];
-  if (active) {
+  // natural(part): the loaded element's part to its place in its line
+  auto natural = [&](auto* all, auto&& part) {
 #pragma unroll
-    for (int q = 0; q < G::J2; ++q) {
-      if (!G::row_ok(t, q)) continue;
+    for (int q = 0; q < PER; ++q) {
+      const int e = threadIdx.x + q * W::NT;
+      if (e < nel) {
+        const int rr = e / (M + 1), k = e - rr * (M + 1);
 #pragma unroll
-      for (int k2 = 0; k2 < G::R2; ++k2) {
-        const int k = t + G::T * q + G::R1 * k2;
-        double2 xk = mine[k], xm = mine[M - k];
-        if (k == 0) { xk.y = 0.0; xm.y = 0.0; }
-        const double er = xk.x + xm.x, ei = xk.y - xm.y;
-        const double dr = xk.x - xm.x, di = xk.y + xm.y;
-        const double2 w = tws[k];
-        const double orr = w.x * dr + w.y * di, oi = w.x * di - w.y * dr;
-        xs[q * G::R2 + k2] = make_double2(er - oi, ei + orr);
+        for (int ff = 0; ff < W::NF; ++ff) all[(size_t)(ff * W::RPB + rr) * Q::LINE + k] = part(v[ff][q]);
       }
     }
-  }
-  __syncthreads();
-  inv_c<M>(xs, xc, mine, t, tw, active);
-  if (active) {
-#pragma unroll
-    for (int j = 0; j < G::J1; ++j)
-      if (G::col_ok(t, j)) {
-#pragma unroll
-        for (int m = 0; m < G::R1; ++m) mine[t + G::T * j + G::R2 * m] = xc[j * G::R1 + m];
-      }
-  }
-  if constexpr (KIND == kPlain) {
     __syncthreads();
-    gptr<double2> out = glb(reinterpret_cast<double2*>(D.out)) + (size_t)row0 * M;
-    for (int e = threadIdx.x; e < nrow * M; e += W::NT) {
-      const int rr = e / M, k = e - rr * M;
-      stc(out + e, lds[(size_t)rr * G::LINE + k]);
-    }
-  } else {
-    double acc[kNSum];
+  };
+  // each(fn): fn(slot, k) for the elements of the thread's rows
+  auto each = [&](auto&& fn) {
+    if (!active) return;
 #pragma unroll
-    for (int k = 0; k < kNSum; ++k) acc[k] = 0.0;
-    fast::x_epi_points<M, KIND, INMODE, OUTMODE, W::RPB, W::NT, 2 * G::LINE, 2 * M, true>(
-        D, reinterpret_cast<const double*>(lds), row0, nrows, 0, acc, outmode);
-    fast::x_epi_sums<OUTMODE>(D, acc, blk);
+    for (int q = 0; q < G::J2; ++q)
+      if (G::row_ok(t, q)) {
+#pragma unroll
+        for (int k2 = 0; k2 < G::R2; ++k2) fn(q * G::R2 + k2, t + G::T * q + G::R1 * k2);
+      }
+  };
+  double acc[kNSum];
+#pragma unroll
+  for (int k = 0; k < kNSum; ++k) acc[k] = 0.0;
+  if constexpr (Q::SC) {
+    double* all = reinterpret_cast<double*>(smem);
+    double* mine = all + (size_t)line * Q::LINE;
+    double er[G::NS], dr[G::NS];
+    natural(all, [](const double2& z) { return z.x; });
+    each([&](int s, int k) {
+      const double a = mine[k], b = mine[M - k];
+      er[s] = a + b;
+      dr[s] = a - b;
+    });
+    __syncthreads();
+    natural(all, [](const double2& z) { return z.y; });
+    each([&](int s, int k) {
+      const double a = k == 0 ? 0.0 : mine[k], b = k == 0 ? 0.0 : mine[M - k];
+      xs[s] = merge(k, er[s], dr[s], a - b, a + b);
+    });
+    __syncthreads();
+    inv_s<M>(xs, xc, mine, t, tw, active);
+    constexpr int H1 = G::R1 / 2;
+    auto half = [&](auto h) {
+      constexpr int H = decltype(h)::value;
+      if (H) __syncthreads();   // the first half's points are read
+      if (active) {
+#pragma unroll
+        for (int j = 0; j < G::J1; ++j)
+          if (G::col_ok(t, j)) {
+#pragma unroll
+            for (int m = 0; m < H1; ++m) {
+              const int i = 2 * (t + G::T * j + G::R2 * m);
+              mine[i] = xc[j * G::R1 + m + H * H1].x;
+              mine[i + 1] = xc[j * G::R1 + m + H * H1].y;
+            }
+          }
+      }
+      if constexpr (KIND == kPlain) {
+        __syncthreads();
+        for (int e = threadIdx.x; e < nrow * M; e += W::NT) {
+          const int rr = e / M, i = e - rr * M;
+          glb(D.out)[(size_t)(row0 + rr) * (2 * M) + H * M + i] = all[(size_t)rr * Q::LINE + i];
+        }
+      } else {
+        fast::x_epi_points<M, KIND, INMODE, OUTMODE, W::RPB, W::NT, Q::LINE, M, true>(D, all, row0, nrows, H * M, acc,
+                                                                                      outmode);
+      }
+    };
+    half(std::integral_constant<int, 0>());
+    half(std::integral_constant<int, 1>());
+  } else {
+    double2* all = reinterpret_cast<double2*>(smem);
+    double2* mine = all + (size_t)line * Q::LINE;
+    natural(all, [](const double2& z) { return z; });
+    each([&](int s, int k) {
+      double2 xk = mine[k], xm = mine[M - k];
+      if (k == 0) { xk.y = 0.0; xm.y = 0.0; }
+      xs[s] = merge(k, xk.x + xm.x, xk.x - xm.x, xk.y - xm.y, xk.y + xm.y);
+    });
+    __syncthreads();
+    inv_c<M>(xs, xc, mine, t, tw, active);
+    if (active) {
+#pragma unroll
+      for (int j = 0; j < G::J1; ++j)
+        if (G::col_ok(t, j)) {
+#pragma unroll
+          for (int m = 0; m < G::R1; ++m) mine[t + G::T * j + G::R2 * m] = xc[j * G::R1 + m];
+        }
+    }
+    if constexpr (KIND == kPlain) {
+      __syncthreads();
+      gptr<double2> out = glb(reinterpret_cast<double2*>(D.out)) + (size_t)row0 * M;
+      for (int e = threadIdx.x; e < nrow * M; e += W::NT) {
+        const int rr = e / M, k = e - rr * M;
+        stc(out + e, all[(size_t)rr * Q::LINE + k]);
+      }
+    } else {
+      fast::x_epi_points<M, KIND, INMODE, OUTMODE, W::RPB, W::NT, 2 * Q::LINE, 2 * M, true>(
+          D, reinterpret_cast<const double*>(all), row0, nrows, 0, acc, outmode);
+    }
   }
+  if constexpr (KIND != kPlain) fast::x_epi_sums<OUTMODE>(D, acc, blk);
 }
 
 // ------------------------------------------------------------ launchers (one translation unit per group)
@@ -746,9 +934,11 @@ template <int M, int KIND>
 static void launch_rows(bool fwd, int inmode, int outmode, const ReqDesc* dd, const GridDims& d, int nb,
                         const double2* tw, const double2* tws, hipStream_t st) {
   using W = RowGeo<M, KIND>;
+  using F = RowGeoF<M, KIND>;
   const dim3 grid(cdiv((long long)d.n2 * d.n3, W::RPB), nb), block(W::NT);
   if (fwd) {
-    hipLaunchKernelGGL((k_rows_fwd<M, KIND>), grid, block, W::LDS, st, dd, d, tw, tws, inmode);
+    allow_lds<k_rows_fwd<M, KIND>>(F::LDS);
+    hipLaunchKernelGGL((k_rows_fwd<M, KIND>), dim3(cdiv((long long)d.n2 * d.n3, F::RPB), nb), dim3(F::NT), F::LDS, st, dd, d, tw, tws, inmode);
   } else if (inmode == kInRho) {
     hipLaunchKernelGGL((k_rows_inv<M, KIND, kInRho, kOutPot>), grid, block, W::LDS, st, dd, d, tw, tws, kOutPot);
   } else if constexpr (KIND != kPlain) {

@@ -145,7 +145,7 @@ int run_eval(const ShapePlan& sp, int kind, int inmode, int outmode, int fp32, c
 int run_finalize(const ShapePlan& sp, int kind, int fp32, const ReqDesc* d_descs, int nb, double* d_sums_out,
                  hipStream_t st);
 // Register-resident fast path (power-of-two WT grids; ofd_fast.hip)
-bool fast_path_ok(const ShapePlan& sp, int kind);
+bool fast_path_ok(const ShapePlan& sp, int kind, int fp32);
 int fast_eval(const ShapePlan& sp, int kind, int inmode, int outmode, int fp32, const ReqDesc* d_descs, int nb,
               hipStream_t st);
 int fast_finalize(const ShapePlan& sp, int kind, int fp32, const ReqDesc* d_descs, int nb, double* out,
@@ -155,6 +155,8 @@ int fast_finalize(const ShapePlan& sp, int kind, int fp32, const ReqDesc* d_desc
 bool gen_path_ok(const ShapePlan& sp);
 int gen_eval(const ShapePlan& sp, int kind, int inmode, int outmode, const ReqDesc* d_descs, int nb, hipStream_t st);
 int gen_partials(const ShapePlan& sp, int kind);
+int gen_rows_inv(const ShapePlan& sp, int kind, int inmode, int outmode, const ReqDesc* d_descs, int nb,
+                 hipStream_t st);
 int gen_fft3d_plain(const ShapePlan& sp, int forward, const ReqDesc* d_descs, int nb, hipStream_t st);
 // Plain 3D transforms of D.u -> D.work (forward, no 1/N) or D.work -> D.out.
 int run_fft3d_plain(const ShapePlan& sp, int forward, const ReqDesc* d_descs, int nb, hipStream_t st);
