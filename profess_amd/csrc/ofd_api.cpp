@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <condition_variable>
 #include <map>
@@ -19,6 +20,7 @@
 #include <new>
 #include <tuple>
 #include <cmath>
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -78,6 +80,65 @@ void stream_put(hipStream_t s) {
   }
   std::lock_guard<std::mutex> lk(g_stream_mu);
   g_streams.push_back(s);
+}
+
+// Pinned host slots of kNSum doubles, one per context, from slabs of 64 KiB
+// that stay with the process (as many as the contexts alive at once need): a
+// context then costs no hipHostMalloc or hipHostFree of its own, which wait
+// for the whole device.
+std::mutex g_slot_mu;
+std::vector<double*> g_slots;
+constexpr size_t kSlotDoubles = 16, kSlabSlots = 512;
+double* slot_get() {
+  std::lock_guard<std::mutex> lk(g_slot_mu);
+  if (g_slots.empty()) {
+    void* p = nullptr;
+    HIPCHK(hipHostMalloc(&p, kSlabSlots * kSlotDoubles * sizeof(double), hipHostMallocDefault));
+    for (size_t i = 0; i < kSlabSlots; ++i) g_slots.push_back(static_cast<double*>(p) + i * kSlotDoubles);
+  }
+  double* s = g_slots.back();
+  g_slots.pop_back();
+  return s;
+}
+void slot_put(double* s) {
+  if (!s) return;
+  std::lock_guard<std::mutex> lk(g_slot_mu);
+  g_slots.push_back(s);
+}
+
+// Waiting for an evaluation's sums. The finalize kernel, the last of an
+// evaluation, stores them into the context's pinned slot as well; the host
+// marks the slot beforehand with a signalling NaN, which no arithmetic leaves
+// behind, and polls until every mark is gone. That is the end of everything
+// the evaluation wrote: the finalize kernel starts when the passes before it
+// have completed and released their stores. Against a copy of the sums and a
+// stream synchronization this saves a copy kernel and the wake-up. After
+// 50 ms, or on a sum that equals the mark, the stream is synchronized as
+// before, which also reports a device error.
+constexpr uint64_t kUnset = 0x7ff4a5c3e1972b6dull;
+static_assert(kNSum <= (int)kSlotDoubles, "a slot holds the sums");
+void mark_sums(double* h) {
+  for (int k = 0; k < kNSum; ++k) __atomic_store_n(reinterpret_cast<uint64_t*>(h) + k, kUnset, __ATOMIC_RELAXED);
+  std::atomic_thread_fence(std::memory_order_seq_cst);
+}
+hipError_t wait_sums(const double* h, hipStream_t st) {
+  const uint64_t* p = reinterpret_cast<const uint64_t*>(h);
+  const auto t0 = std::chrono::steady_clock::now();
+  int k = 0;
+  for (unsigned spin = 1;; ++spin) {
+    while (k < kNSum && __atomic_load_n(p + k, __ATOMIC_ACQUIRE) != kUnset) ++k;
+    if (k == kNSum) return hipSuccess;
+    if (spin % 256 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(50))
+      return hipStreamSynchronize(st);
+    __builtin_ia32_pause();
+  }
+}
+
+// The descriptor travels as a kernel argument: no staging buffer to wait for,
+// and ordered on the stream behind the launches that still read the old one.
+__global__ void k_put_desc(ReqDesc d, ReqDesc* dst) { *dst = d; }
+void put_desc(const ReqDesc& d, ReqDesc* dst, hipStream_t st) {
+  hipLaunchKernelGGL(k_put_desc, dim3(1), dim3(1), 0, st, d, dst);
 }
 
 // A blocking copy ordered on `st` (never on the legacy null stream, which
@@ -350,6 +411,7 @@ struct ofd_ctx {
   void* work = nullptr;      // NF x nc complex (FP64 size)
   double* sums = nullptr;    // partials
   double* fin = nullptr;     // kNSum finalized sums
+  double* hfin = nullptr;    // their pinned host slot (wait_sums)
   double* wgck = nullptr;    // 4 x nc
   double* wtk = nullptr;     // nc: WT kernel coef * LindG / N
   float* wtk32 = nullptr;    // its FP32 copy (precision 1)
@@ -504,6 +566,7 @@ extern "C" int ofd_create(const ofd_grid* g, const ofd_functional* f, double num
     const long long nrows = (long long)g->n2 * g->n3;
     c->sums = dalloc<double>((size_t)nrows * kNSum);
     c->fin = dalloc<double>(kNSum);
+    c->hfin = slot_get();
     if (c->kind == kWGC8) c->wgck = dalloc<double>(4 * nc);
     if (c->kind == kWT3 || c->kind == kWT4) {
       c->wtk = dalloc<double>(nc);
@@ -560,6 +623,7 @@ extern "C" void ofd_destroy(ofd_ctx* c) {
                   (void*)c->many_desc, (void*)c->many_sums, (void*)c->d_frac, (void*)c->d_psp_vqs,
                   (void*)c->d_psp_dd})
     dev_free(b);
+  slot_put(c->hfin);
   graphs_clear(c->graphs);
   if (c->sp.tw_x) shape_plan_free(&c->sp);
   stream_put(c->st);
@@ -615,21 +679,28 @@ static void etable_from_sums(const ofd_ctx* c, const double* s, double* et) {
   etable_calc(s, c->lam, c->mu, c->dV, c->e_ionion, et);
 }
 
-// One evaluation on the context's own descriptor; sums (kNSum) copied back.
-static int eval_one(ofd_ctx* c, const ReqDesc& D, int inmode, int outmode, int fp32, double* h_sums) {
-  if (c->kind == kWGC8 && !c->have_wgc) return fail(c, "WGC kernel table not set (ofd_set_wgc_table)");
-  // stream-ordered upload from the context's own copy, which stays unchanged
-  // until the synchronization below
+// Uploads D as the context's descriptor unless it holds D already.
+static void set_desc(ofd_ctx* c, const ReqDesc& D) {
+  if (std::memcmp(&D, &c->last_desc, sizeof(D)) == 0) return;
   c->last_desc = D;
-  if (hipMemcpyAsync(c->desc, &c->last_desc, sizeof(D), hipMemcpyHostToDevice, c->st) != hipSuccess)
-    return fail(c, "descriptor upload failed");
-  if (launch_eval(c->graphs, c->sp, c->kind, inmode, outmode, fp32, c->desc, 1, c->fin, c->st))
+  put_desc(D, c->desc, c->st);
+}
+
+// One evaluation on the context's own descriptor, complete at return; the sums
+// (kNSum) go to h_sums. Synchronous calls spent 28 us (32^3 to 128^3) to 45 us
+// beside the evaluation's kernels on copying the descriptor in, the sums out
+// and waiting; with the argument-borne descriptor and the polled sums 9 us.
+static int eval_one(ofd_ctx* c, ReqDesc D, int inmode, int outmode, int fp32, double* h_sums) {
+  if (c->kind == kWGC8 && !c->have_wgc) return fail(c, "WGC kernel table not set (ofd_set_wgc_table)");
+  D.hfin = c->hfin;
+  set_desc(c, D);
+  mark_sums(c->hfin);
+  if (launch_eval(c->graphs, c->sp, c->kind, inmode, outmode, fp32, c->desc, 1, c->fin, c->st)) {
+    hipStreamSynchronize(c->st);   // whatever was launched no longer writes the slot
     return fail(c, "kernel launch failed");
-  if (h_sums) {
-    if (hipMemcpyAsync(h_sums, c->fin, kNSum * sizeof(double), hipMemcpyDeviceToHost, c->st) != hipSuccess)
-      return fail(c, "sum copy failed");
   }
-  if (hipStreamSynchronize(c->st) != hipSuccess) return fail(c, "stream synchronize failed");
+  if (wait_sums(c->hfin, c->st) != hipSuccess) return fail(c, "stream synchronize failed");
+  if (h_sums) std::memcpy(h_sums, c->hfin, kNSum * sizeof(double));
   return 0;
 }
 
@@ -651,14 +722,7 @@ extern "C" int ofd_calpot_enqueue(ofd_ctx* c, const double* rho, int opt_sqrt, d
   c->set_rho_io(D, rho, pot);
   D.opt_sqrt = opt_sqrt ? 1 : 0;
   if (sums_dev) D.fin = sums_dev;
-  // the descriptor is uploaded only when it changes, from the context's own
-  // copy (the stream is drained first, so no earlier upload still reads it)
-  if (std::memcmp(&D, &c->last_desc, sizeof(D)) != 0) {
-    if (hipStreamSynchronize(c->st) != hipSuccess) return fail(c, "stream synchronize failed");
-    c->last_desc = D;
-    if (hipMemcpyAsync(c->desc, &c->last_desc, sizeof(D), hipMemcpyHostToDevice, c->st) != hipSuccess)
-      return fail(c, "descriptor upload failed");
-  }
+  set_desc(c, D);
   const int fp32 = c->precision == 1;
   if (launch_eval(c->graphs, c->sp, c->kind, kInRho, kOutPot, fp32, c->desc, 1, sums_dev ? sums_dev : c->fin,
                   c->st))
@@ -683,7 +747,6 @@ constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices] = {};
 
-__global__ void k_put_desc(ReqDesc d, ReqDesc* dst) { *dst = d; }
 __global__ void k_etable_dev(const double* s, double lam, double mu, double dV, double eii, double* et) {
   etable_calc(s, lam, mu, dV, eii, et);
 }
@@ -732,7 +795,7 @@ extern "C" int ofd_calpot_noalloc(ofd_ctx* c, const double* rho, int opt_sqrt, d
   D.sums = reinterpret_cast<double*>(base + off_sums);
   D.work = base + off_work;
   ReqDesc* dd = reinterpret_cast<ReqDesc*>(base);
-  hipLaunchKernelGGL(k_put_desc, dim3(1), dim3(1), 0, c->st, D, dd);
+  put_desc(D, dd, c->st);
   const int fp32 = c->precision == 1;
   if (run_eval(c->sp, c->kind, kInRho, kOutPot, fp32, dd, 1, c->st) ||
       run_finalize(c->sp, c->kind, fp32, dd, 1, D.fin, c->st))
@@ -781,6 +844,7 @@ extern "C" int ofd_calpot_many(ofd_ctx* const* cs, int nb, const double* const* 
       cs[i]->set_rho_io(h[i], rho[i], pot[i]);
       h[i].opt_sqrt = opt_sqrt ? 1 : 0;
       h[i].fin = c0->many_sums + (size_t)i * kNSum;
+      if (ets) h[i].hfin = cs[i]->hfin;
     }
     if (c0->many_last.size() != (size_t)nb ||
         std::memcmp(h.data(), c0->many_last.data(), sizeof(ReqDesc) * nb) != 0) {
@@ -789,14 +853,16 @@ extern "C" int ofd_calpot_many(ofd_ctx* const* cs, int nb, const double* const* 
       HIPCHK(hipMemcpyAsync(c0->many_desc, c0->many_last.data(), sizeof(ReqDesc) * nb, hipMemcpyHostToDevice,
                             c0->st));
     }
+    if (ets)
+      for (int i = 0; i < nb; ++i) mark_sums(cs[i]->hfin);
     const int fp32 = c0->precision == 1;
-    if (launch_eval(c0->graphs, c0->sp, c0->kind, kInRho, kOutPot, fp32, c0->many_desc, nb, c0->many_sums, c0->st))
+    if (launch_eval(c0->graphs, c0->sp, c0->kind, kInRho, kOutPot, fp32, c0->many_desc, nb, c0->many_sums, c0->st)) {
+      hipStreamSynchronize(c0->st);
       return fail(c0, "kernel launch failed");
+    }
     if (ets) {
-      std::vector<double> s((size_t)nb * kNSum);
-      HIPCHK(hipMemcpyAsync(s.data(), c0->many_sums, sizeof(double) * s.size(), hipMemcpyDeviceToHost, c0->st));
-      HIPCHK(hipStreamSynchronize(c0->st));
-      for (int i = 0; i < nb; ++i) etable_from_sums(cs[i], &s[(size_t)i * kNSum], ets + 9 * (size_t)i);
+      for (int i = 0; i < nb; ++i) HIPCHK(wait_sums(cs[i]->hfin, c0->st));
+      for (int i = 0; i < nb; ++i) etable_from_sums(cs[i], cs[i]->hfin, ets + 9 * (size_t)i);
     }
   } catch (const std::exception& e) {
     return fail(c0, e.what());

@@ -25,7 +25,7 @@ __global__ void __launch_bounds__(256) k_fin(const ReqDesc* __restrict__ descs, 
   const ReqDesc& D = descs[blockIdx.y];
   const int k = blockIdx.x;
   gptr<const double> src = glb(D.sums) + (size_t)k * nwg;
-  double acc[1] = {0.0};
+  double acc = 0.0;
   // eight independent loads in flight per thread, summed in a fixed order
   for (int base = 0; base < nwg; base += 8 * 256) {
     double v[8];
@@ -34,9 +34,14 @@ __global__ void __launch_bounds__(256) k_fin(const ReqDesc* __restrict__ descs, 
       const int w = base + threadIdx.x + 256 * j;
       v[j] = w < nwg ? src[w] : 0.0;
     }
-    acc[0] += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    acc += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
   }
-  block_sum_strided<1>(acc, glb(D.fin) + k, 1);
+  __shared__ double red[4];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) put_fin(D, k, ((red[0] + red[1]) + red[2]) + red[3]);
 }
 
 }  // namespace fast

@@ -86,7 +86,15 @@ struct ReqDesc {
   int lsda;        // exchange-correlation of the spin kinds: 1 Perdew-Zunger, 2 Perdew-Wang 92
   int newton_ch;   // kOutNewton with spin kinds: the perturbed channel (0 up, 1 down)
   const float* wtk32;   // FP32 copy of wtk for the FP32 passes (may be null)
+  double* hfin;         // pinned host copy of fin for a caller that waits on it (may be null)
 };
+
+// fin[k] = s, and the host's copy where one is asked for (one 8-byte store
+// across PCIe, whole when it arrives).
+__device__ __forceinline__ void put_fin(const ReqDesc& D, int k, double s) {
+  D.fin[k] = s;
+  if (D.hfin != nullptr) __hip_atomic_store(D.hfin + k, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 struct GridDims {
   int n1, n2, n3;

@@ -529,7 +529,7 @@ __global__ void __launch_bounds__(256) k_finalize(const ReqDesc* __restrict__ de
   for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
   __syncthreads();
-  if (threadIdx.x == 0) D.fin[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+  if (threadIdx.x == 0) put_fin(D, blockIdx.x, (red[0] + red[1]) + (red[2] + red[3]));
 }
 
 // ============================================================ host launchers
