@@ -2903,6 +2903,10 @@ extern "C" int ofd_autotune(ofd_ctx* c, int reps, ofd_tune_result* res) {
       cx = {0};
       cp = {1};
     }
+    if (yz_path_ok(c->sp, c->kind, fp32)) {   // no y pass; the z pass's tile
+      cy = {};
+      cz = {1, 2, 4};
+    }
     cy.insert(cy.begin(), 0);
     cz.insert(cz.begin(), 0);
     ShapePlan& sp = c->sp;

@@ -46,7 +46,8 @@ __global__ void __launch_bounds__(256) k_fin(const ReqDesc* __restrict__ descs, 
 
 }  // namespace fast
 
-// FP32: every shape of the line lengths below. FP64: the shapes of the
+// FP32: every shape of the line lengths below. FP64, of what the three-pass
+// evaluations (ofd_yz.hip, asked first) leave: the shapes of the
 // power-of-two plane passes (32 x 32, 64 x 64, 128 x 128), where two fused
 // passes beat the general form's three: Wang-Teter / fast against general
 // passes, 32^3 20.7 / 21.9 us, 64^3 34.5 / 35.3, 128^3 96 / 109. The general

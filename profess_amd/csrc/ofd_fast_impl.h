@@ -1006,23 +1006,34 @@ __device__ __forceinline__ double epi32(const ReqDesc& D, double rho_d, double v
 // chunk's loads are issued before the workgroup barrier that completes the
 // lines in LDS (this function starts with that barrier). The sums go to acc.
 // FM: field j of row rr sits at line j*RPB + rr instead (field-major lines).
-// OUTMODE -1: the form is the run-time `outmode`.
+// OUTMODE -1: the form is the run-time `outmode`. RPB 0: the rows, threads and
+// the distance between rows come from `dyn`, with at most 20 / NF points per
+// thread (up to 10 rows, and at least NF (M + 1) threads).
+struct DynRows {
+  int rows = 0, threads = 0, step = 1;
+};
 template <int M, int KIND, int INMODE, int OUTMODE, int RPB, int NT, int LR, int PPR, bool FM = false, typename R>
 __device__ __forceinline__ void x_epi_points(const ReqDesc& D, const R* __restrict__ lr, long long row0,
-                                             long long nrows, int ioff, double (&acc)[kNSum], int outmode = OUTMODE) {
+                                             long long nrows, int ioff, double (&acc)[kNSum], int outmode = OUTMODE,
+                                             DynRows dyn = DynRows{}) {
   constexpr int NF = NF_<KIND>::v;
-  constexpr int EPT = (RPB * PPR + NT - 1) / NT;
+  constexpr bool DYN = RPB == 0;
+  constexpr int EPT = DYN ? (20 + NF - 1) / NF : (RPB * PPR + NT - 1) / (DYN ? 1 : NT);
+  const int nt = DYN ? dyn.threads : NT, rpb = DYN ? dyn.rows : RPB;
   // global loads per point: u and vion, v (trial points and the optimizer
   // forms), b and w (Newton form); at most 16 doubles in flight per thread
   constexpr int NL = 2 + (INMODE == kInPhi || OUTMODE != kOutPot ? 1 : 0) +
                      (OUTMODE == kOutNewton || OUTMODE < 0 ? 2 : 0);
   const int om = OUTMODE >= 0 ? OUTMODE : outmode;
   constexpr int PF = EPT < 16 / NL ? EPT : 16 / NL;
-  const int nrow = (int)min((long long)RPB, nrows - row0);
+  const int nrow = DYN ? rpb : (int)min((long long)RPB, nrows - row0);
   const int npts = nrow * PPR;
   const size_t gbase = (size_t)row0 * 2 * M + ioff;
   // global index of the workgroup's point e (row e / PPR, point e % PPR + ioff)
-  auto gidx = [&](int e) { return PPR == 2 * M ? gbase + e : gbase + (size_t)(e / PPR) * 2 * M + e % PPR; };
+  auto gidx = [&](int e) {
+    if constexpr (DYN) return gbase + (size_t)(e / PPR) * dyn.step * 2 * M + e % PPR;
+    else return PPR == 2 * M ? gbase + e : gbase + (size_t)(e / PPR) * 2 * M + e % PPR;
+  };
   // the second vector: the phi direction of a trial point (kInPhi), the
   // search direction of the signed form, the CG direction of the Newton form
   const bool want_v = D.v != nullptr && (INMODE == kInPhi || om != kOutPot);
@@ -1033,7 +1044,7 @@ __device__ __forceinline__ void x_epi_points(const ReqDesc& D, const R* __restri
     for (int q = 0; q < PF; ++q) {
       // points past the workgroup's last read its last point (in bounds, no
       // branch between the loads) and are not computed
-      const size_t g = gidx(min((int)threadIdx.x + (c0 + q) * NT, npts - 1));
+      const size_t g = gidx(min((int)threadIdx.x + (c0 + q) * nt, npts - 1));
       pv[q] = pb[q] = pw[q] = 0.0;
       pu[q] = glb(D.u)[g];
       if (want_v) pv[q] = glb(D.v)[g];
@@ -1054,13 +1065,13 @@ __device__ __forceinline__ void x_epi_points(const ReqDesc& D, const R* __restri
     }
 #pragma unroll
     for (int q = 0; q < PF; ++q) {
-      const int e = threadIdx.x + (c0 + q) * NT;
+      const int e = threadIdx.x + (c0 + q) * nt;
       if (c0 + q >= EPT || e >= npts) break;
       const int rr = e / PPR, ii = e - rr * PPR;
       const size_t g = gidx(e);
       double o[NF];
 #pragma unroll
-      for (int j = 0; j < NF; ++j) o[j] = (double)lr[(size_t)(FM ? j * RPB + rr : rr * NF + j) * LR + ii];
+      for (int j = 0; j < NF; ++j) o[j] = (double)lr[(size_t)(FM ? j * rpb + rr : rr * NF + j) * LR + ii];
       if constexpr (is_spin_kind(KIND)) {
         // both channels: the second one's inputs are loaded here
         double t1 = 0.0, t2 = 0.0, r1, r2;

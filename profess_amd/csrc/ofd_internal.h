@@ -166,6 +166,11 @@ int gen_partials(const ShapePlan& sp, int kind);
 int gen_rows_inv(const ShapePlan& sp, int kind, int inmode, int outmode, const ReqDesc* d_descs, int nb,
                  hipStream_t st);
 int gen_fft3d_plain(const ShapePlan& sp, int forward, const ReqDesc* d_descs, int nb, hipStream_t st);
+// FP64 evaluations in three passes, the y transform divided between x and z
+// (ofd_yz.hip)
+bool yz_path_ok(const ShapePlan& sp, int kind, int fp32);
+int yz_eval(const ShapePlan& sp, int kind, int inmode, int outmode, const ReqDesc* d_descs, int nb, hipStream_t st);
+int yz_partials(const ShapePlan& sp, int kind);
 // Plain 3D transforms of D.u -> D.work (forward, no 1/N) or D.work -> D.out.
 int run_fft3d_plain(const ShapePlan& sp, int forward, const ReqDesc* d_descs, int nb, hipStream_t st);
 

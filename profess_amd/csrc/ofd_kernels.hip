@@ -600,6 +600,7 @@ static bool use_gen(const ShapePlan& sp, int fp32) { return !sp.force_generic &&
 
 int run_eval(const ShapePlan& sp, int kind, int inmode, int outmode, int fp32, const ReqDesc* dd, int nb,
              hipStream_t st) {
+  if (yz_path_ok(sp, kind, fp32)) return yz_eval(sp, kind, inmode, outmode, dd, nb, st);
   if (!sp.force_generic && fast_path_ok(sp, kind, fp32)) return fast_eval(sp, kind, inmode, outmode, fp32, dd, nb, st);
   if (use_gen(sp, fp32)) return gen_eval(sp, kind, inmode, outmode, dd, nb, st);
   return fp32 ? eval_r<float>(sp, kind, inmode, outmode, dd, nb, st)
@@ -607,11 +608,12 @@ int run_eval(const ShapePlan& sp, int kind, int inmode, int outmode, int fp32, c
 }
 
 int run_finalize(const ShapePlan& sp, int kind, int fp32, const ReqDesc* dd, int nb, double* out, hipStream_t st) {
-  if (!sp.force_generic && fast_path_ok(sp, kind, fp32)) return fast_finalize(sp, kind, fp32, dd, nb, out, st);
+  const bool yz = yz_path_ok(sp, kind, fp32);
+  if (!yz && !sp.force_generic && fast_path_ok(sp, kind, fp32)) return fast_finalize(sp, kind, fp32, dd, nb, out, st);
   const Tiles t = tiles_for(sp, func_nf(kind), fp32 ? (int)sizeof(float2) : (int)sizeof(double2));
   (void)out;
   hipLaunchKernelGGL(k_finalize, dim3(kNSum, nb), dim3(256), 0, st, dd,
-                     use_gen(sp, fp32) ? gen_partials(sp, kind) : t.ntile);
+                     yz ? yz_partials(sp, kind) : use_gen(sp, fp32) ? gen_partials(sp, kind) : t.ntile);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

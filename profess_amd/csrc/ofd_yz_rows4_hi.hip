@@ -1,0 +1,16 @@
+// Row passes (x with the inner part of y) of kWT4 for one group of lengths (ofd_yz_impl.h).
+#include "ofd_yz_impl.h"
+
+namespace ofd {
+namespace yz {
+template <> YzRowsFn yz_rows_hi<kWT4>(int m) {
+  switch (m) {
+#define X(N, A, B, T_) \
+  case N: return launch_rows<N, kWT4>;
+    OFD_YZ_ROWS_HI(X)
+#undef X
+    default: return nullptr;
+  }
+}
+}  // namespace yz
+}  // namespace ofd
