@@ -22,7 +22,7 @@ SOURCES = ["ofd_kernels.hip", "ofd_fast.hip", "ofd_fast_d3.hip", "ofd_fast_d4.hi
 # the general FP64 passes: columns by group of lengths, rows by field count and group
 SOURCES += ["ofd_gen_cols_%s.hip" % g for g in "abcde"]
 SOURCES += ["ofd_yz.hip", "ofd_yz_cols_a.hip", "ofd_yz_cols_b.hip", "ofd_yz_rows3_lo.hip", "ofd_yz_rows3_hi.hip",
-            "ofd_yz_rows4_lo.hip", "ofd_yz_rows4_hi.hip"]
+            "ofd_yz_rows4_lo.hip", "ofd_yz_rows4_hi.hip", "ofd_yz_rows5_lo.hip", "ofd_yz_rows5_hi.hip"]
 SOURCES += ["ofd_gen_rows%s_%s.hip" % (k, g) for k in "134578" for g in ("lo", "hi")]
 COMMON = ["-std=c++17", "-O3", "-fPIC", "-pthread", "-Wno-unused-result", "-Wno-unused-value"]
 DEVICE = ["--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

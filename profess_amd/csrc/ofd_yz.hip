@@ -7,12 +7,18 @@ template <> YzRowsFn yz_rows_lo<kWT3>(int);
 template <> YzRowsFn yz_rows_hi<kWT3>(int);
 template <> YzRowsFn yz_rows_lo<kWT4>(int);
 template <> YzRowsFn yz_rows_hi<kWT4>(int);
+template <> YzRowsFn yz_rows_lo<kWT3S>(int);
+template <> YzRowsFn yz_rows_hi<kWT3S>(int);
 
 static YzFn z_of(int n) { return n < 54 ? yz_a(n) : yz_b(n); }
+template <int KIND> static YzRowsFn rows_k(int m) { return m < 54 ? yz_rows_lo<KIND>(m) : yz_rows_hi<KIND>(m); }
 static YzRowsFn rows_of(int kind, int m) {
-  if (kind == kWT3) return m < 54 ? yz_rows_lo<kWT3>(m) : yz_rows_hi<kWT3>(m);
-  if (kind == kWT4) return m < 54 ? yz_rows_lo<kWT4>(m) : yz_rows_hi<kWT4>(m);
-  return nullptr;
+  switch (kind) {
+    case kWT3: return rows_k<kWT3>(m);
+    case kWT4: return rows_k<kWT4>(m);
+    case kWT3S: return rows_k<kWT3S>(m);
+    default: return nullptr;
+  }
 }
 // lanes per row of a half length M and per column of a z length
 static int row_lanes(int m) {
@@ -36,18 +42,19 @@ static bool is_a(int r) { return false OFD_YZ_A(OFD_YZ_IS); }
 #undef OFD_YZ_IS
 
 // The split of the shape's y length and the tiles, or A = 0 where the five
-// passes stay: WGC (its z pass couples the fields), two spin channels (90^3
-// 79 / 78 us of kernels) and FP32; an x workgroup of more than 256 lanes (five
+// passes stay: WGC (its z pass couples the fields), FP32, two spin channels on
+// the 32 x 32 planes (which keep the plane passes' bits) or with alpha != beta
+// (7 fields: 80 x 75 x 63 115 / 90 us, 90 x 75 x 96 150 / 129); an x workgroup of more than 256 lanes (five
 // waves share a CU badly: 108 x 72 x 108 with four fields and 288 lanes
 // 94.5 / 89.4 us a call; at 240 to 256 lanes 96 x 64 x 96 56 / 82, 128^3
 // 147 / 161), z columns of more than 256 lanes, and y lengths without two
-// factors A, B of 3..16 and 3..10 within a factor of two (75 = 15 x 5 in
-// 100 x 75 x 81 with four fields: 56 / 51 us of kernels). Synchronous calls
+// factors A, B of 4..16 and 3..10 within a factor of three. Synchronous calls
 // against the five passes (for 32^3, 64^3 and 128^3 the plane passes), alpha =
 // beta / alpha != beta: 32^3 26.3 / 28.4 and 29.7 / 32.5, 72^3 44.1 / 52.7 and
 // 60.7 / 70.9, 100^3 66.6 / 79.2 and 82.6 / 99.4, 128^3 96.4 / 103.2 and
-// 147 / 161, 150^3 172 / 197 and 264 / 275; over 110 random shapes of 18 to
-// 160 points an axis none lost more than the runs differ.
+// 147 / 161, 150^3 172 / 197 and 264 / 275, 100 x 75 x 81 62 / 77 and 73 / 87;
+// two channels 90^3 89 / 97; over 230 random shapes of 18 to 160 points an axis
+// none lost more than the runs differ.
 // A z workgroup takes the widest tile of at most four waves. An x-forward
 // workgroup takes one field (100^3 14.4 us, all three 17.5) unless its M + 1
 // elements then leave a second wave nearly empty (128^3 28.7, all three 22.9)
@@ -55,12 +62,12 @@ static bool is_a(int r) { return false OFD_YZ_A(OFD_YZ_IS); }
 static YZ plan(const ShapePlan& sp, int kind) {
   const GridDims& d = sp.d;
   YZ g{};
-  if (kind != kWT3 && kind != kWT4) return g;
+  if (kind == kWGC8 || kind == kWT4S || (kind == kWT3S && fast_path_ok(sp, kind, 0))) return g;
   const int nf = func_nf(kind), tx = row_lanes(d.M), tz = col_lanes(d.n3);
-  if (tx == 0 || tz == 0) return g;
+  if (tx == 0 || tz == 0 || nf * (d.M + 1) > 512) return g;
   for (int b = 10; b >= 3; --b) {
     const int a = d.n2 / b;
-    if (a * b != d.n2 || a < b || a > 2 * b || !is_a(a)) continue;
+    if (a * b != d.n2 || a < b || a > 3 * b || !is_a(a)) continue;
     if (b * nf * tx > 256 || std::max(a * tz, d.n3) > 256) return g;
     g.A = a;
     g.B = b;

@@ -19,11 +19,12 @@ from tests.test_gpu_lengths import LAT, _run, pa  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 GRIDS = [(18, 16, 16), (20, 18, 28), (24, 25, 105), (36, 112, 126), (128, 32, 18), (126, 28, 20), (100, 100, 24),
-         (42, 128, 30), (28, 160, 16), (120, 50, 27), (54, 81, 120), (30, 49, 128), (192, 42, 150), (162, 63, 27)]
+         (42, 128, 30), (28, 160, 16), (120, 50, 27), (54, 81, 120), (30, 49, 128), (192, 42, 150), (162, 63, 27), (60, 75, 24),
+         (36, 21, 63)]
 
 
 @pytest.mark.parametrize("grid", GRIDS)
-@pytest.mark.parametrize("kind", ["wt", "wt4"])
+@pytest.mark.parametrize("kind", ["wt", "wt4", "spin"])
 def test_three_pass(pa, monkeypatch, grid, kind):  # noqa: F811
     print(grid, kind, flush=True)
     n1, n2, n3 = grid
@@ -33,6 +34,8 @@ def test_three_pass(pa, monkeypatch, grid, kind):  # noqa: F811
     rng = np.random.default_rng(n1 + 7 * n2 + 31 * n3)
     rho = 0.027 * (1.0 + 0.3 * (2.0 * rng.random(cell.shape) - 1.0))
     vion = rng.random(cell.shape) - 0.5
+    if kind == "spin":
+        rho = np.stack([0.55 * rho, 0.45 * rho[::-1]])
     pot, et = _run(pa, grid, kind, rho, vion, ne, lat)
     monkeypatch.setenv("OFD_GENERIC", "1")
     p0, e0 = _run(pa, grid, kind, rho, vion, ne, lat)
@@ -41,7 +44,7 @@ def test_three_pass(pa, monkeypatch, grid, kind):  # noqa: F811
     assert np.all(np.abs(et - e0) <= 1e-12 * np.abs(e0) + 1e-12)
     f = O.Functional(kinetic=4, alpha=0.9 if kind == "wt4" else -100.0, beta=0.7 if kind == "wt4" else -100.0)
     sysm = O.System(cell, f.resolve(ne, cell.vol), vion)
-    ref, er = O.calculate_potential_plus(rho, sysm)
+    ref, er = (O.calculate_potential_plus_spin if kind == "spin" else O.calculate_potential_plus)(rho, sysm)
     assert np.max(np.abs(pot - ref)) <= 1e-10 * np.max(np.abs(ref))
     assert np.all(np.abs(et - er) <= 1e-10 * np.abs(er) + 1e-12)
 
