@@ -472,7 +472,7 @@ def main():
                    "grid": [n, n, n], "atoms": len(case["frac"]), "batch": 1},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": read_traffic(),
-                     "kernel": "one evaluation (5 fused passes + partial-sum finalize)",
+                     "kernel": "one evaluation (3 fused passes at 128^3, otherwise 3 to 5, + partial-sum finalize)",
                      "algorithmic_bytes": bw},
     }
     if args.batch > 1:
