@@ -509,28 +509,40 @@ __global__ void __launch_bounds__(256) k_xinv(const ReqDesc* __restrict__ descs,
 // ------------------------------------------------------------ finalize: sum partials
 // One workgroup per (slot, request): fin[slot] = sum of the workgroup
 // partials (laid out [slot][workgroup]), eight independent loads in flight
-// per thread, fixed order.
-__global__ void __launch_bounds__(256) k_finalize(const ReqDesc* __restrict__ descs, int nwg) {
+// per thread, fixed order. Bound by the chain of rounds of 8 NT partials, each
+// a trip to memory; NT is finalize_threads().
+template <int NT>
+__global__ void __launch_bounds__(NT) k_finalize(const ReqDesc* __restrict__ descs, int nwg) {
   const ReqDesc& D = descs[blockIdx.y];
   const double* src = D.sums + (size_t)blockIdx.x * nwg;
-  double acc[1] = {0.0};
-  for (int base = 0; base < nwg; base += 8 * 256) {
+  double x = 0.0;
+  for (int base = 0; base < nwg; base += 8 * NT) {
     double v[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int w = base + threadIdx.x + 256 * j;
+      const int w = base + threadIdx.x + NT * j;
       v[j] = w < nwg ? src[w] : 0.0;
     }
-    acc[0] += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    x += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
   }
-  __shared__ double red[4];
-  double x = acc[0];
+  __shared__ double red[NT / 64];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
   __syncthreads();
-  if (threadIdx.x == 0) put_fin(D, blockIdx.x, (red[0] + red[1]) + (red[2] + red[3]));
+  if (threadIdx.x == 0) {
+    double s[NT / 256];
+#pragma unroll
+    for (int k = 0; k < NT / 256; ++k) s[k] = (red[4 * k] + red[4 * k + 1]) + (red[4 * k + 2] + red[4 * k + 3]);
+    if constexpr (NT == 256) put_fin(D, blockIdx.x, s[0]);
+    else put_fin(D, blockIdx.x, (s[0] + s[1]) + (s[2] + s[3]));
+  }
 }
+
+// 1024 threads where 256 would take three rounds or more: 256^3 WT (32768
+// partials) 986.6 -> 982.9 us a call, WGC (65536) 2613.5 -> 2606.6, 200^3 within
+// noise; up to 4096 partials (128^3: 2048) the 256 threads stay.
+static int finalize_threads(int nwg) { return nwg > 4096 ? 1024 : 256; }
 
 // ============================================================ host launchers
 template <typename R>
@@ -612,8 +624,9 @@ int run_finalize(const ShapePlan& sp, int kind, int fp32, const ReqDesc* dd, int
   if (!yz && !sp.force_generic && fast_path_ok(sp, kind, fp32)) return fast_finalize(sp, kind, fp32, dd, nb, out, st);
   const Tiles t = tiles_for(sp, func_nf(kind), fp32 ? (int)sizeof(float2) : (int)sizeof(double2));
   (void)out;
-  hipLaunchKernelGGL(k_finalize, dim3(kNSum, nb), dim3(256), 0, st, dd,
-                     yz ? yz_partials(sp, kind) : use_gen(sp, fp32) ? gen_partials(sp, kind) : t.ntile);
+  const int nwg = yz ? yz_partials(sp, kind) : use_gen(sp, fp32) ? gen_partials(sp, kind) : t.ntile;
+  if (finalize_threads(nwg) == 1024) hipLaunchKernelGGL(k_finalize<1024>, dim3(kNSum, nb), dim3(1024), 0, st, dd, nwg);
+  else hipLaunchKernelGGL(k_finalize<256>, dim3(kNSum, nb), dim3(256), 0, st, dd, nwg);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
