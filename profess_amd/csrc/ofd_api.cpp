@@ -137,8 +137,9 @@ hipError_t wait_sums(const double* h, hipStream_t st) {
 // The descriptor travels as a kernel argument: no staging buffer to wait for,
 // and ordered on the stream behind the launches that still read the old one.
 __global__ void k_put_desc(ReqDesc d, ReqDesc* dst) { *dst = d; }
-void put_desc(const ReqDesc& d, ReqDesc* dst, hipStream_t st) {
+int put_desc(const ReqDesc& d, ReqDesc* dst, hipStream_t st) {
   hipLaunchKernelGGL(k_put_desc, dim3(1), dim3(1), 0, st, d, dst);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 // A blocking copy ordered on `st` (never on the legacy null stream, which
@@ -416,7 +417,7 @@ struct ofd_ctx {
   double* wtk = nullptr;     // nc: WT kernel coef * LindG / N
   float* wtk32 = nullptr;    // its FP32 copy (precision 1)
   ReqDesc* desc = nullptr;   // one descriptor
-  ReqDesc last_desc{};       // what `desc` holds after an enqueue
+  ReqDesc last_desc{};       // what `desc` holds after an enqueue; zero: not known
   ReqDesc* many_desc = nullptr;
   double* many_sums = nullptr;
   int many_cap = 0;
@@ -477,6 +478,7 @@ static int fail(ofd_ctx* c, const std::string& m) {
   if (c) c->err = m;
   return -1;
 }
+static void forget_desc(ofd_ctx* c) { std::memset(&c->last_desc, 0, sizeof(c->last_desc)); }
 
 // Inverse-transpose of the lattice (long double), G vectors rb = 2 pi A^{-T}
 // (CellInfo.f90:281), volume |det A| (MathFunctions Volume).
@@ -679,11 +681,14 @@ static void etable_from_sums(const ofd_ctx* c, const double* s, double* et) {
   etable_calc(s, c->lam, c->mu, c->dV, c->e_ionion, et);
 }
 
-// Uploads D as the context's descriptor unless it holds D already.
-static void set_desc(ofd_ctx* c, const ReqDesc& D) {
-  if (std::memcmp(&D, &c->last_desc, sizeof(D)) == 0) return;
+// Uploads D as the context's descriptor unless it holds D already. After a
+// failed upload or launch nothing is known of what it holds.
+static int set_desc(ofd_ctx* c, const ReqDesc& D) {
+  if (std::memcmp(&D, &c->last_desc, sizeof(D)) == 0) return 0;
+  forget_desc(c);
+  if (put_desc(D, c->desc, c->st)) return fail(c, "descriptor upload failed");
   c->last_desc = D;
-  put_desc(D, c->desc, c->st);
+  return 0;
 }
 
 // One evaluation on the context's own descriptor, complete at return; the sums
@@ -693,13 +698,17 @@ static void set_desc(ofd_ctx* c, const ReqDesc& D) {
 static int eval_one(ofd_ctx* c, ReqDesc D, int inmode, int outmode, int fp32, double* h_sums) {
   if (c->kind == kWGC8 && !c->have_wgc) return fail(c, "WGC kernel table not set (ofd_set_wgc_table)");
   D.hfin = c->hfin;
-  set_desc(c, D);
+  if (set_desc(c, D)) return -1;
   mark_sums(c->hfin);
   if (launch_eval(c->graphs, c->sp, c->kind, inmode, outmode, fp32, c->desc, 1, c->fin, c->st)) {
     hipStreamSynchronize(c->st);   // whatever was launched no longer writes the slot
+    forget_desc(c);
     return fail(c, "kernel launch failed");
   }
-  if (wait_sums(c->hfin, c->st) != hipSuccess) return fail(c, "stream synchronize failed");
+  if (wait_sums(c->hfin, c->st) != hipSuccess) {
+    forget_desc(c);
+    return fail(c, "stream synchronize failed");
+  }
   if (h_sums) std::memcpy(h_sums, c->hfin, kNSum * sizeof(double));
   return 0;
 }
@@ -722,11 +731,13 @@ extern "C" int ofd_calpot_enqueue(ofd_ctx* c, const double* rho, int opt_sqrt, d
   c->set_rho_io(D, rho, pot);
   D.opt_sqrt = opt_sqrt ? 1 : 0;
   if (sums_dev) D.fin = sums_dev;
-  set_desc(c, D);
+  if (set_desc(c, D)) return -1;
   const int fp32 = c->precision == 1;
   if (launch_eval(c->graphs, c->sp, c->kind, kInRho, kOutPot, fp32, c->desc, 1, sums_dev ? sums_dev : c->fin,
-                  c->st))
+                  c->st)) {
+    forget_desc(c);
     return fail(c, "kernel launch failed");
+  }
   return 0;
 }
 
@@ -795,7 +806,7 @@ extern "C" int ofd_calpot_noalloc(ofd_ctx* c, const double* rho, int opt_sqrt, d
   D.sums = reinterpret_cast<double*>(base + off_sums);
   D.work = base + off_work;
   ReqDesc* dd = reinterpret_cast<ReqDesc*>(base);
-  put_desc(D, dd, c->st);
+  if (put_desc(D, dd, c->st)) return fail(c, "descriptor upload failed");
   const int fp32 = c->precision == 1;
   if (run_eval(c->sp, c->kind, kInRho, kOutPot, fp32, dd, 1, c->st) ||
       run_finalize(c->sp, c->kind, fp32, dd, 1, D.fin, c->st))
@@ -858,6 +869,7 @@ extern "C" int ofd_calpot_many(ofd_ctx* const* cs, int nb, const double* const* 
     const int fp32 = c0->precision == 1;
     if (launch_eval(c0->graphs, c0->sp, c0->kind, kInRho, kOutPot, fp32, c0->many_desc, nb, c0->many_sums, c0->st)) {
       hipStreamSynchronize(c0->st);
+      c0->many_last.clear();
       return fail(c0, "kernel launch failed");
     }
     if (ets) {
@@ -865,6 +877,7 @@ extern "C" int ofd_calpot_many(ofd_ctx* const* cs, int nb, const double* const* 
       for (int i = 0; i < nb; ++i) etable_from_sums(cs[i], cs[i]->hfin, ets + 9 * (size_t)i);
     }
   } catch (const std::exception& e) {
+    c0->many_last.clear();   // the copy it stands for may not have been made
     return fail(c0, e.what());
   }
   return 0;
@@ -2103,7 +2116,7 @@ extern "C" int ofd_set_spin(ofd_ctx* c, const ofd_spin* sp) {
       }
     }
     graphs_clear(c->graphs);
-    std::memset(&c->last_desc, 0, sizeof(c->last_desc));
+    forget_desc(c);
     c->many_last.clear();
     c->kind = kind;
     c->nspin = sp->nspin;
@@ -2852,6 +2865,7 @@ static double time_current(ofd_ctx* c, int reps) {
   D.out = c->pot;
   D.opt_sqrt = 1;
   HIPCHK(hipStreamSynchronize(c->st));
+  forget_desc(c);
   HIPCHK(copy_sync(c->desc, &D, sizeof(D), hipMemcpyHostToDevice, c->st));
   c->last_desc = D;
   const int fp32 = c->precision == 1;
@@ -2939,7 +2953,7 @@ extern "C" int ofd_autotune(ofd_ctx* c, int reps, ofd_tune_result* res) {
                                                                              sp.no_plane ? 1 : 0};
     }
     graphs_clear(c->graphs);
-    std::memset(&c->last_desc, 0, sizeof(c->last_desc));
+    forget_desc(c);
     if (res) {
       res->rows_x = sp.rows_x;
       res->kb_y = sp.kb_y;

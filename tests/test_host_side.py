@@ -1,0 +1,88 @@
+"""The library's host side on a HIP runtime of the host alone (hip_stub.hip):
+what is launched and uploaded, no numbers. Each case runs in a process of its
+own, where the stub's symbols come before the HIP runtime's."""
+import os
+import shutil
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIPCC = os.environ.get("HIPCC") or shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+
+PREAMBLE = """
+import ctypes as C, os, sys
+import numpy as np
+stub = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+stub.stub_listed.restype = C.c_char_p
+for f in ("u", "out", "u2", "out2"):
+    getattr(stub, "stub_" + f).restype = C.c_void_p
+import profess_amd as pa
+from profess_amd import calpot
+L = pa.lib()
+
+def system(grid, spin=False, **kw):
+    s = pa.OFDSystem(np.diag(0.4 * np.array(grid)), grid, 21.0, **kw)
+    if spin:
+        s.set_spin(2)
+    return s
+
+def enqueue(s, rho, pot):   # device addresses: no kernel runs that would read them
+    return L.ofd_calpot_enqueue(s._h, C.c_void_p(rho), 1, C.c_void_p(pot), None)
+
+def device(s, rho, pot):   # the synchronous call; nothing writes the sums, so it ends by its 50 ms
+    return L.ofd_calpot_device(s._h, C.c_void_p(rho), 1, C.c_void_p(pot), None)
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    if not os.path.exists(os.path.join(ROOT, "profess_amd", "libprofess_amd.so")):
+        pytest.skip("library not built")
+    so = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
+    subprocess.run([HIPCC, "-x", "hip", "--cuda-host-only", "-std=c++17", "-O1", "-fPIC", "-shared", "-o", so,
+                    os.path.join(ROOT, "tests", "hip_stub.hip")], check=True)
+
+    def go(code):
+        r = subprocess.run([sys.executable, "-c", PREAMBLE + textwrap.dedent(code), so], cwd=ROOT,
+                           capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+        return r.stdout
+    return go
+
+
+@pytest.mark.parametrize("call", ["enqueue", "device"])
+def test_failed_descriptor_upload_is_repeated(run, call):
+    """A call whose descriptor did not reach the device fails, and the same
+    call made again uploads it: the pass reads the second call's pointers."""
+    run(f"""
+    s = system((24, 24, 24))
+    assert {call}(s, 4096, 8192) == 0 and stub.stub_u() == 4096
+    stub.stub_fail(b"k_put_desc")
+    assert {call}(s, 12288, 16384) != 0
+    stub.stub_fail(b"")
+    assert {call}(s, 12288, 16384) == 0
+    assert (stub.stub_u(), stub.stub_out()) == (12288, 16384)
+    """)
+
+
+def test_failed_batch_upload_is_repeated(run):
+    """As above for the descriptors of a batched call, which are copied."""
+    run("""
+    s = [system((24, 24, 24)) for _ in range(2)]
+    def many(rho, pot):
+        return calpot.CalculatePotentialPlusMany(s, [rho, rho + 4096], [pot, pot + 4096], eTable=False)
+    many(4096, 65536)
+    assert stub.stub_u() == 4096
+    stub.stub_fail(b"hipMemcpyAsync")
+    try:
+        many(16384, 131072)
+        assert False
+    except calpot.OFDError:
+        pass
+    stub.stub_fail(b"")
+    many(16384, 131072)
+    assert (stub.stub_u(), stub.stub_out()) == (16384, 131072)
+    """)
