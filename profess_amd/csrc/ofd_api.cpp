@@ -685,6 +685,12 @@ static void etable_from_sums(const ofd_ctx* c, const double* s, double* et) {
 // failed upload or launch nothing is known of what it holds.
 static int set_desc(ofd_ctx* c, const ReqDesc& D) {
   if (std::memcmp(&D, &c->last_desc, sizeof(D)) == 0) return 0;
+  // Recorded into a caller's capture, the upload would not run now and would
+  // run, unseen, at every replay. ofd_calpot_noalloc carries a descriptor of
+  // its own there.
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c->st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
+    return fail(c, "new arguments while the stream is captured (ofd_calpot_noalloc can be captured)");
   forget_desc(c);
   if (put_desc(D, c->desc, c->st)) return fail(c, "descriptor upload failed");
   c->last_desc = D;

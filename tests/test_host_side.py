@@ -86,3 +86,21 @@ def test_failed_batch_upload_is_repeated(run):
     many(16384, 131072)
     assert (stub.stub_u(), stub.stub_out()) == (16384, 131072)
     """)
+
+
+@pytest.mark.parametrize("call", ["enqueue", "device"])
+def test_new_arguments_are_refused_under_capture(run, call):
+    """A call that needs its descriptor uploaded is refused while the stream is
+    captured and launches nothing; made again afterwards it is uploaded. The
+    form for captures is not refused."""
+    run(f"""
+    s = system((24, 24, 24))
+    assert {call}(s, 4096, 8192) == 0
+    stub.stub_capture(1)
+    stub.stub_clear()
+    assert {call}(s, 12288, 16384) != 0 and stub.stub_listed() == b""
+    assert L.ofd_calpot_noalloc(s._h, C.c_void_p(4096), 1, C.c_void_p(8192), None) == 0
+    stub.stub_capture(0)
+    assert {call}(s, 12288, 16384) == 0
+    assert (stub.stub_u(), stub.stub_out()) == (12288, 16384)
+    """)
