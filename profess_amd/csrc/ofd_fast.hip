@@ -57,9 +57,10 @@ __global__ void __launch_bounds__(256) k_fin(const ReqDesc* __restrict__ descs, 
 bool fast_path_ok(const ShapePlan& sp, int kind, int fp32) {
   if (!fast_path_ok_impl(sp, kind)) return false;
   if (fp32) return true;
+  // the FP64 chain has no forward passes but the plane's, so it takes a shape
+  // only where the plane fits in LDS
   const int M = sp.d.M;
-  const bool plane = !sp.no_plane && (M == 16 || M == 32 || M == 64) && sp.d.n2 == 2 * M && !is_gp_len(sp.d.n3);
-  if (!plane) return false;
+  if ((M != 16 && M != 32 && M != 64) || is_gp_len(sp.d.n3) || !plane_for<double>(sp)) return false;
   return kind == kWGC8 ? M == 64 : (!is_spin_kind(kind) || M == 16);
 }
 

@@ -1857,7 +1857,7 @@ template <typename R> static inline bool plane_for(const ShapePlan& sp) {
 // the x-inverse pass still waits for both branches, and the smaller launches
 // of each branch lose what the overlap gains.)
 template <typename R, int KIND, int INMODE, int OUTMODE, int M>
-static void fast_chain(const ShapePlan& sp, const FastTiles& ft, const ReqDesc* dd, int nb, hipStream_t st,
+static int fast_chain(const ShapePlan& sp, const FastTiles& ft, const ReqDesc* dd, int nb, hipStream_t st,
                        const typename V2<R>::T* twx, const typename V2<R>::T* tws, const typename V2<R>::T* twy,
                        const typename V2<R>::T* twz) {
   constexpr int NF = fast::NF_<KIND>::v;
@@ -1901,7 +1901,8 @@ static void fast_chain(const ShapePlan& sp, const FastTiles& ft, const ReqDesc* 
   if constexpr (sizeof(R) == 8) {
     // the plane shapes only (fast_path_ok)
     const int pl = try_plane<R, KIND, INMODE>(sp, dd, nb, st, twx, tws, twy, 0, NF);
-    zlaunch(st, pl > 1 ? pl : 1, 0, NF);
+    if (pl == 0) return -1;
+    zlaunch(st, pl, 0, NF);
     launch_y<R, 2 * M, +1>(sp, ft.kby, 0, NF, dd, nb, st, twy);
     if (gen_inverse(sp, 0)) gen_rows_inv(sp, KIND, INMODE, OUTMODE, dd, nb, st);
     else if constexpr (M < 64) launch_x<R, M, KIND, INMODE, OUTMODE>(sp, ft, dd, nb, st, false, twx, tws);
@@ -1919,6 +1920,7 @@ static void fast_chain(const ShapePlan& sp, const FastTiles& ft, const ReqDesc* 
     ylaunch(std::integral_constant<int, +1>(), st, 0, NF);
     launch_x<R, M, KIND, INMODE, OUTMODE>(sp, ft, dd, nb, st, false, twx, tws);
   }
+  return 0;
 }
 
 template <typename R, int KIND, int INMODE, int OUTMODE>
@@ -1932,28 +1934,29 @@ static int fast_eval_t(const ShapePlan& sp, const ReqDesc* dd, int nb, hipStream
     twx = sp.tw_x; tws = sp.tw_s; twy = sp.tw_y; twz = sp.tw_z;
   }
   (void)f32;
+  int rc = 0;
   if constexpr (sizeof(R) == 8) {   // the plane shapes
     switch (sp.d.M) {
-      case 16: fast_chain<R, KIND, INMODE, OUTMODE, 16>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-      case 32: fast_chain<R, KIND, INMODE, OUTMODE, 32>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-      default: fast_chain<R, KIND, INMODE, OUTMODE, 64>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 16: rc = fast_chain<R, KIND, INMODE, OUTMODE, 16>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 32: rc = fast_chain<R, KIND, INMODE, OUTMODE, 32>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      default: rc = fast_chain<R, KIND, INMODE, OUTMODE, 64>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
     }
   } else {
     switch (sp.d.M) {
-      case 16: fast_chain<R, KIND, INMODE, OUTMODE, 16>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-      case 24: fast_chain<R, KIND, INMODE, OUTMODE, 24>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-      case 32: fast_chain<R, KIND, INMODE, OUTMODE, 32>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-      case 40: fast_chain<R, KIND, INMODE, OUTMODE, 40>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-      case 48: fast_chain<R, KIND, INMODE, OUTMODE, 48>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-      case 60: fast_chain<R, KIND, INMODE, OUTMODE, 60>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-      case 96: fast_chain<R, KIND, INMODE, OUTMODE, 96>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-      case 120: fast_chain<R, KIND, INMODE, OUTMODE, 120>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-      case 64: fast_chain<R, KIND, INMODE, OUTMODE, 64>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-      case 128: fast_chain<R, KIND, INMODE, OUTMODE, 128>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-      default: fast_chain<R, KIND, INMODE, OUTMODE, 256>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 16: rc = fast_chain<R, KIND, INMODE, OUTMODE, 16>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 24: rc = fast_chain<R, KIND, INMODE, OUTMODE, 24>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 32: rc = fast_chain<R, KIND, INMODE, OUTMODE, 32>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 40: rc = fast_chain<R, KIND, INMODE, OUTMODE, 40>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 48: rc = fast_chain<R, KIND, INMODE, OUTMODE, 48>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 60: rc = fast_chain<R, KIND, INMODE, OUTMODE, 60>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 96: rc = fast_chain<R, KIND, INMODE, OUTMODE, 96>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 120: rc = fast_chain<R, KIND, INMODE, OUTMODE, 120>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 64: rc = fast_chain<R, KIND, INMODE, OUTMODE, 64>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      case 128: rc = fast_chain<R, KIND, INMODE, OUTMODE, 128>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      default: rc = fast_chain<R, KIND, INMODE, OUTMODE, 256>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
     }
   }
-  return hipGetLastError() == hipSuccess ? 0 : -1;
+  return rc == 0 && hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 template <typename R, int KIND>

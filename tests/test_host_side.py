@@ -27,10 +27,18 @@ def system(grid, spin=False, **kw):
     s = pa.OFDSystem(np.diag(0.4 * np.array(grid)), grid, 21.0, **kw)
     if spin:
         s.set_spin(2)
+    if kw.get("kinetic") == 5:
+        s.set_wgc_table(*[np.linspace(0.01, 5.0, 50)] * 4)
     return s
 
 def enqueue(s, rho, pot):   # device addresses: no kernel runs that would read them
     return L.ofd_calpot_enqueue(s._h, C.c_void_p(rho), 1, C.c_void_p(pot), None)
+
+def passes(s):   # "family kernel" of each launch of one evaluation
+    import re
+    stub.stub_clear()
+    assert enqueue(s, 4096, 8192) == 0
+    return [" ".join(m) for m in re.findall(r"_ZN3ofd(?:\\d(fast|gen|yz))?\\d+(\\w+?)(?:I|E)", stub.stub_listed().decode())]
 
 def device(s, rho, pot):   # the synchronous call; nothing writes the sums, so it ends by its 50 ms
     return L.ofd_calpot_device(s._h, C.c_void_p(rho), 1, C.c_void_p(pot), None)
@@ -103,4 +111,16 @@ def test_new_arguments_are_refused_under_capture(run, call):
     stub.stub_capture(0)
     assert {call}(s, 12288, 16384) == 0
     assert (stub.stub_u(), stub.stub_out()) == (12288, 16384)
+    """)
+
+
+@pytest.mark.parametrize("grid,kinetic", [((128, 128, 192), 4), ((128, 128, 24), 5)])
+@pytest.mark.parametrize("lds", [65536, 131072, 163840])
+def test_plane_passes_only_where_the_plane_fits(run, grid, kinetic, lds):
+    """Every evaluation starts with a forward pass over x, also where a
+    workgroup has less LDS than the 128 x 128 plane (157 KB whole) takes."""
+    run(f"""
+    stub.stub_lds({lds})
+    p = passes(system({grid}, kinetic={kinetic}))
+    assert p[0] == ("fast k_plane_fwd" if {lds} == 163840 else "gen k_rows_fwd"), p
     """)
