@@ -40,6 +40,13 @@ def passes(s):   # "family kernel" of each launch of one evaluation
     assert enqueue(s, 4096, 8192) == 0
     return [" ".join(m) for m in re.findall(r"_ZN3ofd(?:\\d(fast|gen|yz))?\\d+(\\w+?)(?:I|E)", stub.stub_listed().decode())]
 
+FAMILY = {"yz k_rows_fwd": "three", "fast k_plane_fwd": "plane", "gen k_rows_fwd": "general"}
+OPTS = {"wt4": dict(alpha=0.9, beta=0.7), "spin4": dict(alpha=0.9, beta=0.7), "wgc": dict(kinetic=5)}
+
+def family(grid, kind):   # the passes that an FP64 evaluation takes
+    p = passes(system(grid, spin=kind.startswith("spin"), **OPTS.get(kind, {})))
+    return next((FAMILY[x] for x in p if x in FAMILY), "staged")
+
 def device(s, rho, pot):   # the synchronous call; nothing writes the sums, so it ends by its 50 ms
     return L.ofd_calpot_device(s._h, C.c_void_p(rho), 1, C.c_void_p(pot), None)
 """
@@ -123,4 +130,18 @@ def test_plane_passes_only_where_the_plane_fits(run, grid, kinetic, lds):
     stub.stub_lds({lds})
     p = passes(system({grid}, kinetic={kinetic}))
     assert p[0] == ("fast k_plane_fwd" if {lds} == 163840 else "gen k_rows_fwd"), p
+    """)
+
+
+def test_shapes_reach_the_passes_they_test(run):
+    """The shapes of the tests of one family of FP64 passes against another
+    take that family, so that no change of the dispatch empties a test."""
+    run("""
+    from tests import test_gpu_lengths as lengths, test_gpu_plane_fp64 as plane, test_gpu_three_pass as three
+    want = [(g, k, "plane") for g, k in plane.CASES]
+    want += [(g, k, "general") for g in lengths.GRIDS for k in ("wt", "wt4", "spin", "wgc")
+             if g != (100, 75, 81) or k == "wgc"]
+    want += [(g, k, "three") for g in three.GRIDS for k in ("wt", "wt4", "spin") if (g, k) != ((162, 63, 27), "spin")]
+    got = [(g, k, family(g, k)) for g, k, _ in want]
+    assert got == want, [(a, b[2]) for a, b in zip(got, want) if a != b]
     """)
