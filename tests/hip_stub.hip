@@ -40,6 +40,8 @@ API void stub_clear() { listed.clear(); }
 API const char* stub_listed() { return listed.c_str(); }
 API unsigned stub_host_flags() { return host_flags; }
 // fields of the descriptor the last evaluation pass was given
+API const ofd::ReqDesc* stub_desc() { return desc; }
+API int stub_sizes(int k) { return k == 0 ? sizeof(ofd::ReqDesc) : sizeof(ofd::ShapePlan); }
 API const void* stub_u() { return desc->u; }
 API const void* stub_out() { return desc->out; }
 API const void* stub_u2() { return desc->u2; }

@@ -138,10 +138,28 @@ def test_shapes_reach_the_passes_they_test(run):
     take that family, so that no change of the dispatch empties a test."""
     run("""
     from tests import test_gpu_lengths as lengths, test_gpu_plane_fp64 as plane, test_gpu_three_pass as three
+    from tests import test_gpu_forms as forms
     want = [(g, k, "plane") for g, k in plane.CASES]
     want += [(g, k, "general") for g in lengths.GRIDS for k in ("wt", "wt4", "spin", "wgc")
              if g != (100, 75, 81) or k == "wgc"]
     want += [(g, k, "three") for g in three.GRIDS for k in ("wt", "wt4", "spin") if (g, k) != ((162, 63, 27), "spin")]
+    want += forms.CASES
     got = [(g, k, family(g, k)) for g, k, _ in want]
     assert got == want, [(a, b[2]) for a, b in zip(got, want) if a != b]
+    """)
+
+
+def test_descriptor_layout_of_the_form_tests(run):
+    """The descriptor that the tests of single forms fill is the library's."""
+    run("""
+    from tests.eval_forms import PLAN_BYTES, ReqDesc
+    stub.stub_desc.restype = C.POINTER(ReqDesc)
+    assert C.sizeof(ReqDesc) == stub.stub_sizes(0) and PLAN_BYTES >= stub.stub_sizes(1)
+    s = system((24, 24, 24), spin=True, alpha=0.9, beta=0.7)
+    assert enqueue(s, 4096, 8192) == 0
+    D = stub.stub_desc().contents
+    n = 8 * 24 ** 3
+    assert (D.u, D.out, D.u2, D.out2) == (4096, 8192, 4096 + n, 8192 + n)
+    assert (D.alpha, D.beta, D.opt_sqrt, D.lsda, D.pad, D.newton_ch, D.cb2, D.hfin) == (0.9, 0.7, 1, 1, 0, 0, 0.0, None)
+    assert abs(D.rb[0] - 2 * np.pi / 9.6) < 1e-12 and D.wtk and D.fin and D.work and D.sums and D.vion
     """)
