@@ -2867,8 +2867,7 @@ extern "C" int ofd_ion_relax(ofd_ctx* c, double* rhoR, double* frac_xyz, const o
 // untuned one.
 static double time_current(ofd_ctx* c, int reps) {
   ReqDesc D = c->base_desc();
-  D.u = c->rho;
-  D.out = c->pot;
+  c->set_rho_io(D, c->rho, c->pot);
   D.opt_sqrt = 1;
   HIPCHK(hipStreamSynchronize(c->st));
   forget_desc(c);
@@ -2899,8 +2898,8 @@ extern "C" int ofd_autotune(ofd_ctx* c, int reps, ofd_tune_result* res) {
   if (!c) return -1;
   if (reps < 1) reps = 5;
   try {
-    const long long n = c->nr();
-    std::vector<double> h(n, c->num_ele / c->vol);
+    const long long n = c->nr_all();
+    std::vector<double> h(n, c->num_ele / c->vol / c->nspin);
     HIPCHK(copy_sync(c->rho, h.data(), n * sizeof(double), hipMemcpyHostToDevice, c->st));
     graphs_clear(c->graphs);
     const bool fast = !c->sp.force_generic && fast_path_ok(c->sp, c->kind, c->precision == 1);

@@ -163,3 +163,18 @@ def test_descriptor_layout_of_the_form_tests(run):
     assert (D.alpha, D.beta, D.opt_sqrt, D.lsda, D.pad, D.newton_ch, D.cb2, D.hfin) == (0.9, 0.7, 1, 1, 0, 0, 0.0, None)
     assert abs(D.rb[0] - 2 * np.pi / 9.6) < 1e-12 and D.wtk and D.fin and D.work and D.sums and D.vion
     """)
+
+
+def test_autotune_evaluates_both_channels(run):
+    """The evaluations that the tuner times have the arrays of both channels."""
+    run("""
+    from tests.eval_forms import ReqDesc
+    stub.stub_desc.restype = C.POINTER(ReqDesc)
+    s = system((24, 24, 24), spin=True)
+    s.autotune(reps=1)
+    D = stub.stub_desc().contents
+    n = 24 ** 3
+    assert (D.u2, D.out2) == (D.u + 8 * n, D.out + 8 * n)
+    rho = np.ctypeslib.as_array(C.cast(D.u, C.POINTER(C.c_double)), (2 * n,))
+    assert np.all(np.abs(rho * 2 * s.vol / 21.0 - 1.0) < 1e-12)
+    """)
