@@ -375,7 +375,8 @@ typedef struct ofd_tune_result {
   double us_best;     /* one evaluation with the chosen tiles */
 } ofd_tune_result;
 /* Times `reps` evaluations per candidate tile shape on the context's stream
- * (coordinate descent over plane pass, z tiles, y tiles, x rows), keeps the
+ * (coordinate descent over z tiles and y tiles; the passes and a result's bits
+ * stay), keeps the
  * fastest in the context and records it for every context created later
  * with the same grid, functional kind and precision. */
 int ofd_autotune(ofd_ctx* ctx, int reps, ofd_tune_result* out);

@@ -379,7 +379,7 @@ struct TuneKey {
   }
 };
 struct TuneChoice {
-  int rows_x, kb_y, kb_z, no_plane;
+  int rows_x, kb_y, kb_z;
 };
 static std::mutex g_tune_mu;
 static std::map<TuneKey, TuneChoice> g_tuned;
@@ -591,7 +591,6 @@ extern "C" int ofd_create(const ofd_grid* g, const ofd_functional* f, double num
         c->sp.rows_x = it->second.rows_x;
         c->sp.kb_y = it->second.kb_y;
         c->sp.kb_z = it->second.kb_z;
-        c->sp.no_plane = it->second.no_plane != 0;
       }
     }
   } catch (const std::exception& e) {
@@ -2904,15 +2903,11 @@ extern "C" int ofd_autotune(ofd_ctx* c, int reps, ofd_tune_result* res) {
     graphs_clear(c->graphs);
     const bool fast = !c->sp.force_generic && fast_path_ok(c->sp, c->kind, c->precision == 1);
     const int fp32 = c->precision == 1;
-    std::vector<int> cy, cz, cx, cp;
+    std::vector<int> cy, cz, cx;
     if (fast) {
       cy = fast_tile_candidates(c->sp, c->kind, fp32, 1);
       cz = fast_tile_candidates(c->sp, c->kind, fp32, 2);
       cx = {0};
-      // the fused plane pass stays as the plan has it: it reaches the same
-      // result as the separate passes only to rounding (different contraction
-      // of the split's products), and tuning must never change a result's bits
-      cp = {c->sp.no_plane ? 1 : 0};
     } else {
       // the x rows per workgroup set how the energy partials are grouped, so
       // they stay fixed: tuning never changes a result's bits
@@ -2920,7 +2915,6 @@ extern "C" int ofd_autotune(ofd_ctx* c, int reps, ofd_tune_result* res) {
       cy = gen ? std::vector<int>{8, 16, 24, 32} : std::vector<int>{1, 2, 4, 8, 16};
       cz = gen ? cy : std::vector<int>{1, 2, 4, 8};
       cx = {0};
-      cp = {1};
     }
     if (yz_path_ok(c->sp, c->kind, fp32)) {   // no y pass; the z pass's tile
       cy = {};
@@ -2930,12 +2924,15 @@ extern "C" int ofd_autotune(ofd_ctx* c, int reps, ofd_tune_result* res) {
     cz.insert(cz.begin(), 0);
     ShapePlan& sp = c->sp;
     sp.rows_x = 0; sp.kb_y = 0; sp.kb_z = 0;
-    if (cp.size() == 1) sp.no_plane = cp[0] != 0;
+    // the plane pass stays as the plan has it: it reaches the same result as the
+    // other passes only to rounding (different contraction of the split's
+    // products), and tuning must never change a result's bits, here or, with
+    // other spin channels, later
     const double t_def = time_current(c, reps);
     double best = t_def;
     int tried = 1;
     // coordinate descent, one dimension at a time
-    int cur_plane = sp.no_plane ? 1 : 0, cur_z = 0, cur_y = 0, cur_x = 0;
+    int cur_z = 0, cur_y = 0, cur_x = 0;
     auto run_dim = [&](std::vector<int>& cand, int& cur, auto set) {
       int bestv = cur;
       for (int v : cand) {
@@ -2948,14 +2945,13 @@ extern "C" int ofd_autotune(ofd_ctx* c, int reps, ofd_tune_result* res) {
       cur = bestv;
       set(bestv);
     };
-    run_dim(cp, cur_plane, [&](int v) { sp.no_plane = v != 0; });
     run_dim(cz, cur_z, [&](int v) { sp.kb_z = v; });
     run_dim(cy, cur_y, [&](int v) { sp.kb_y = v; });
     if (!fast) run_dim(cx, cur_x, [&](int v) { sp.rows_x = v; });
     {
       std::lock_guard<std::mutex> lk(g_tune_mu);
-      g_tuned[TuneKey{sp.d.n1, sp.d.n2, sp.d.n3, c->kind, fp32}] = TuneChoice{sp.rows_x, sp.kb_y, sp.kb_z,
-                                                                             sp.no_plane ? 1 : 0};
+      g_tuned[TuneKey{sp.d.n1, sp.d.n2, sp.d.n3, c->kind, fp32}] =
+          TuneChoice{sp.rows_x, sp.kb_y, sp.kb_z};
     }
     graphs_clear(c->graphs);
     forget_desc(c);
@@ -3065,7 +3061,6 @@ extern "C" int ofd_pool_create(int n1, int n2, int n3, int capacity, int kinetic
       p->sp.rows_x = it->second.rows_x;
       p->sp.kb_y = it->second.kb_y;
       p->sp.kb_z = it->second.kb_z;
-      p->sp.no_plane = it->second.no_plane != 0;
     }
   }
   if (hipStreamCreateWithFlags(&p->st, hipStreamNonBlocking) != hipSuccess ||

@@ -43,9 +43,11 @@ def passes(s):   # "family kernel" of each launch of one evaluation
 FAMILY = {"yz k_rows_fwd": "three", "fast k_plane_fwd": "plane", "gen k_rows_fwd": "general"}
 OPTS = {"wt4": dict(alpha=0.9, beta=0.7), "spin4": dict(alpha=0.9, beta=0.7), "wgc": dict(kinetic=5)}
 
-def family(grid, kind):   # the passes that an FP64 evaluation takes
-    p = passes(system(grid, spin=kind.startswith("spin"), **OPTS.get(kind, {})))
-    return next((FAMILY[x] for x in p if x in FAMILY), "staged")
+def family_of(s):   # the passes that an FP64 evaluation takes
+    return next((FAMILY[x] for x in passes(s) if x in FAMILY), "staged")
+
+def family(grid, kind):
+    return family_of(system(grid, spin=kind.startswith("spin"), **OPTS.get(kind, {})))
 
 def device(s, rho, pot):   # the synchronous call; nothing writes the sums, so it ends by its 50 ms
     return L.ofd_calpot_device(s._h, C.c_void_p(rho), 1, C.c_void_p(pot), None)
@@ -177,4 +179,24 @@ def test_autotune_evaluates_both_channels(run):
     assert (D.u2, D.out2) == (D.u + 8 * n, D.out + 8 * n)
     rho = np.ctypeslib.as_array(C.cast(D.u, C.POINTER(C.c_double)), (2 * n,))
     assert np.all(np.abs(rho * 2 * s.vol / 21.0 - 1.0) < 1e-12)
+    """)
+
+
+@pytest.mark.parametrize("grid,kind", [((64, 64, 256), "spin"), ((64, 64, 256), "wt"), ((32, 32, 24), "wgc"),
+                                       ((200, 27, 20), "wt"), ((24, 24, 24), "wt"), ((16, 16, 16), "wt")])
+def test_tuning_keeps_the_passes(run, grid, kind):
+    """A tuned system takes the passes it took before, also with one channel
+    again after two, and so does the next system of its shape: another family
+    would change a result's last bits."""
+    run(f"""
+    grid, kind = {grid}, "{kind}"
+    one = family(grid, kind.replace("spin", "wt"))
+    before = family(grid, kind)
+    s = system(grid, spin=kind == "spin", **OPTS.get(kind, {{}}))
+    s.autotune(reps=1)
+    assert family_of(s) == before
+    if kind == "spin":
+        s.set_spin(1)
+        assert family_of(s) == one, family_of(s)
+    assert family(grid, kind) == before and family(grid, kind.replace("spin", "wt")) == one
     """)
