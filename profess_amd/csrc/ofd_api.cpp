@@ -2916,7 +2916,8 @@ extern "C" int ofd_autotune(ofd_ctx* c, int reps, ofd_tune_result* res) {
       cz = gen ? cy : std::vector<int>{1, 2, 4, 8};
       cx = {0};
     }
-    if (yz_path_ok(c->sp, c->kind, fp32)) {   // no y pass; the z pass's tile
+    const bool yz = yz_path_ok(c->sp, c->kind, fp32);
+    if (yz) {   // no y pass; the z pass's tile
       cy = {};
       cz = {1, 2, 4};
     }
@@ -2959,7 +2960,7 @@ extern "C" int ofd_autotune(ofd_ctx* c, int reps, ofd_tune_result* res) {
       res->rows_x = sp.rows_x;
       res->kb_y = sp.kb_y;
       res->kb_z = sp.kb_z;
-      res->plane = sp.no_plane ? 0 : 1;
+      res->plane = !yz && fast && fast_plane_available(sp, fp32) ? 1 : 0;
       res->configs_tried = tried;
       res->us_default = t_def;
       res->us_best = best;

@@ -94,21 +94,7 @@ std::vector<int> fast_tile_candidates(const ShapePlan& sp, int kind, int fp32, i
   return out;
 }
 
-bool fast_plane_available(const ShapePlan& sp, int kind, int fp32) {
-  (void)kind;
-  const int cb = fp32 ? (int)sizeof(float2) : (int)sizeof(double2);
-  auto fits = [&](int M, int N2) {
-    const int S = std::max(M + M / p2_R1(M), M + 1);
-    return (long long)(N2 + N2 / p2_R1(N2)) * S * cb <= sp.lds_cap;
-  };
-  if (sp.d.M == 64 && sp.d.n2 == 128) return fits(64, 128);
-  if (sp.d.M == 32 && sp.d.n2 == 64) return fits(32, 64);
-  if (sp.d.M == 16 && sp.d.n2 == 32) return fits(16, 32);
-  if (sp.d.M == 48 && sp.d.n2 == 96) return fits(48, 96);
-  if (sp.d.M == 40 && sp.d.n2 == 80) return fits(40, 80);
-  if (sp.d.M == 24 && sp.d.n2 == 48) return fits(24, 48);
-  return false;
-}
+bool fast_plane_available(const ShapePlan& sp, int fp32) { return fp32 ? plane_for<float>(sp) : plane_for<double>(sp); }
 
 // Sums the x-inverse pass's per-workgroup partials into each request's fin.
 int fast_finalize(const ShapePlan& sp, int kind, int fp32, const ReqDesc* dd, int nb, double*, hipStream_t st) {

@@ -190,7 +190,7 @@ void vec_scale_sign(double* y, const double* x, const double* s, long long n, hi
 // wavefronts within the LDS limit.
 std::vector<int> fast_tile_candidates(const ShapePlan& sp, int kind, int fp32, int which);
 // Whether the fused x+y plane pass exists for this shape and fits in LDS.
-bool fast_plane_available(const ShapePlan& sp, int kind, int fp32);
+bool fast_plane_available(const ShapePlan& sp, int fp32);
 
 // Batched vector operations over many requests of one grid size.
 enum VecOpKind : int { kOpLincomb = 0, kOpAxpby = 1, kOpZero = 2, kOpCG = 3 };

@@ -200,3 +200,13 @@ def test_tuning_keeps_the_passes(run, grid, kind):
         assert family_of(s) == one, family_of(s)
     assert family(grid, kind) == before and family(grid, kind.replace("spin", "wt")) == one
     """)
+
+
+@pytest.mark.parametrize("grid,kw", [((128, 128, 128), {}), ((128, 128, 192), {}), ((128, 128, 128), dict(precision=1)),
+                                     ((120, 120, 120), dict(precision=1)), ((200, 27, 20), {}), ((16, 16, 16), {})])
+def test_tuner_reports_the_plane_pass(run, grid, kw):
+    run(f"""
+    s = system({grid}, **{kw})
+    p = passes(s)
+    assert s.autotune(reps=1)["plane"] == int("fast k_plane_fwd" in p), p
+    """)
