@@ -379,10 +379,19 @@ struct TuneKey {
   }
 };
 struct TuneChoice {
-  int rows_x, kb_y, kb_z;
+  int kb_y, kb_z;
 };
 static std::mutex g_tune_mu;
 static std::map<TuneKey, TuneChoice> g_tuned;
+static void take_tuned(ShapePlan& sp, int kind) {
+  std::lock_guard<std::mutex> lk(g_tune_mu);
+  for (int fp32 = 0; fp32 < 2; ++fp32) {
+    auto it = g_tuned.find(TuneKey{sp.d.n1, sp.d.n2, sp.d.n3, kind, fp32});
+    if (it == g_tuned.end()) continue;
+    sp.kb_y[fp32] = it->second.kb_y;
+    sp.kb_z[fp32] = it->second.kb_z;
+  }
+}
 
 // ====================================================================== context
 struct ofd_ctx {
@@ -584,15 +593,7 @@ extern "C" int ofd_create(const ofd_grid* g, const ofd_functional* f, double num
     c->dot_part = dalloc<double>(512 * 4);
     c->dot_out = dalloc<double>(4);
     HIPCHK(hipStreamSynchronize(c->st));   // later calls may copy on other streams
-    {
-      std::lock_guard<std::mutex> lk(g_tune_mu);
-      auto it = g_tuned.find(TuneKey{g->n1, g->n2, g->n3, c->kind, c->precision == 1 ? 1 : 0});
-      if (it != g_tuned.end()) {
-        c->sp.rows_x = it->second.rows_x;
-        c->sp.kb_y = it->second.kb_y;
-        c->sp.kb_z = it->second.kb_z;
-      }
-    }
+    take_tuned(c->sp, c->kind);
   } catch (const std::exception& e) {
     c->err = e.what();
     *out = c;
@@ -2924,7 +2925,9 @@ extern "C" int ofd_autotune(ofd_ctx* c, int reps, ofd_tune_result* res) {
     cy.insert(cy.begin(), 0);
     cz.insert(cz.begin(), 0);
     ShapePlan& sp = c->sp;
-    sp.rows_x = 0; sp.kb_y = 0; sp.kb_z = 0;
+    sp.rows_x = 0;
+    int &kb_y = sp.kb_y[fp32], &kb_z = sp.kb_z[fp32];
+    kb_y = kb_z = 0;
     // the plane pass stays as the plan has it: it reaches the same result as the
     // other passes only to rounding (different contraction of the split's
     // products), and tuning must never change a result's bits, here or, with
@@ -2946,20 +2949,19 @@ extern "C" int ofd_autotune(ofd_ctx* c, int reps, ofd_tune_result* res) {
       cur = bestv;
       set(bestv);
     };
-    run_dim(cz, cur_z, [&](int v) { sp.kb_z = v; });
-    run_dim(cy, cur_y, [&](int v) { sp.kb_y = v; });
+    run_dim(cz, cur_z, [&](int v) { kb_z = v; });
+    run_dim(cy, cur_y, [&](int v) { kb_y = v; });
     if (!fast) run_dim(cx, cur_x, [&](int v) { sp.rows_x = v; });
     {
       std::lock_guard<std::mutex> lk(g_tune_mu);
-      g_tuned[TuneKey{sp.d.n1, sp.d.n2, sp.d.n3, c->kind, fp32}] =
-          TuneChoice{sp.rows_x, sp.kb_y, sp.kb_z};
+      g_tuned[TuneKey{sp.d.n1, sp.d.n2, sp.d.n3, c->kind, fp32}] = TuneChoice{kb_y, kb_z};
     }
     graphs_clear(c->graphs);
     forget_desc(c);
     if (res) {
       res->rows_x = sp.rows_x;
-      res->kb_y = sp.kb_y;
-      res->kb_z = sp.kb_z;
+      res->kb_y = kb_y;
+      res->kb_z = kb_z;
       res->plane = !yz && fast && fast_plane_available(sp, fp32) ? 1 : 0;
       res->configs_tried = tried;
       res->us_default = t_def;
@@ -3055,15 +3057,7 @@ extern "C" int ofd_pool_create(int n1, int n2, int n3, int capacity, int kinetic
     *out = p;
     return -1;
   }
-  {
-    std::lock_guard<std::mutex> lk(g_tune_mu);
-    auto it = g_tuned.find(TuneKey{n1, n2, n3, kWT3, precision == 1 ? 1 : 0});
-    if (it != g_tuned.end()) {
-      p->sp.rows_x = it->second.rows_x;
-      p->sp.kb_y = it->second.kb_y;
-      p->sp.kb_z = it->second.kb_z;
-    }
-  }
+  take_tuned(p->sp, kWT3);
   if (hipStreamCreateWithFlags(&p->st, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreateWithFlags(&p->ev_phase, hipEventDisableTiming) != hipSuccess ||
       hipMalloc(&p->d_desc, sizeof(ReqDesc) * rows) != hipSuccess ||

@@ -1649,10 +1649,11 @@ static inline FastTiles fast_tiles(const ShapePlan& sp, int cbytes) {
   const int wy = 64 / Ty, wz = 64 / Tz;
   const long long ly = col_line_bytes(sp.d.n2, cbytes, 1),
                   lz = col_line_bytes(sp.d.n3, cbytes, 2);
-  const long long ty = sp.kb_y > 0 ? sp.lds_cap : tgt, tz = sp.kb_z > 0 ? sp.lds_cap : tgt;
-  ft.kby = sp.kb_y > 0 ? std::max(wy, sp.kb_y / wy * wy) : 256 / Ty;
+  const int ky = sp.kb_y[cbytes == sizeof(float2)], kz = sp.kb_z[cbytes == sizeof(float2)];
+  const long long ty = ky > 0 ? sp.lds_cap : tgt, tz = kz > 0 ? sp.lds_cap : tgt;
+  ft.kby = ky > 0 ? std::max(wy, ky / wy * wy) : 256 / Ty;
   while (ft.kby > wy && (ft.kby * ly > ty || ft.kby * Ty > 256)) ft.kby -= wy;
-  ft.kbz = sp.kb_z > 0 ? std::max(wz, sp.kb_z / wz * wz) : 256 / Tz;
+  ft.kbz = kz > 0 ? std::max(wz, kz / wz * wz) : 256 / Tz;
   while (ft.kbz > wz && (ft.kbz * lz > tz || ft.kbz * Tz > 256)) ft.kbz -= wz;
   return ft;
 }
@@ -1759,7 +1760,7 @@ static void launch_z(const ShapePlan& sp, int kb, const ReqDesc* dd, int nb, hip
     // (the one-component z exchange: half the LDS per column, so a whole
     // 256-thread workgroup of columns unless the tuner picked a tile)
     const int kbj = P > 1 ? std::max(P, kb / P * P)
-                          : (fz_scalar<N, R, 1>() && sp.kb_z <= 0 ? 256 / P2<N>::R2 : kb);
+                          : (fz_scalar<N, R, 1>() && sp.kb_z[sizeof(R) == 4] <= 0 ? 256 / P2<N>::R2 : kb);
     const long long ngrp = (long long)sp.d.K1 * (sp.d.n2 / P);
     const dim3 grid((unsigned)((ngrp + kbj / P - 1) / (kbj / P)), fn, nb), block(kbj * P2<N>::R2);
     const size_t lds = (size_t)kbj * col_stride<N>() * sizeof(C);

@@ -62,9 +62,9 @@ int gen_eval(const ShapePlan& sp, int kind, int inmode, int outmode, const ReqDe
   const ColFns cy = cols_of(d.n2), cz = cols_of(d.n3);
   const int nf = func_nf(kind);
   rows(true, inmode, outmode, dd, d, nb, sp.tw_x, sp.tw_s, st);
-  cy.cols(-1, dd, d.nc, y_cols(d), nf, nb, sp.kb_y, sp.tw_y, st);
-  cz.z(kind, dd, d, nb, sp.kb_z, sp.tw_z, st);
-  cy.cols(+1, dd, d.nc, y_cols(d), nf, nb, sp.kb_y, sp.tw_y, st);
+  cy.cols(-1, dd, d.nc, y_cols(d), nf, nb, sp.kb_y[0], sp.tw_y, st);
+  cz.z(kind, dd, d, nb, sp.kb_z[0], sp.tw_z, st);
+  cy.cols(+1, dd, d.nc, y_cols(d), nf, nb, sp.kb_y[0], sp.tw_y, st);
   rows(false, inmode, outmode, dd, d, nb, sp.tw_x, sp.tw_s, st);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }

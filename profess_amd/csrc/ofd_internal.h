@@ -119,10 +119,11 @@ struct ShapePlan {
   float2* tw_z32 = nullptr;
   float2* tw_s32 = nullptr;
   // launch shapes: 0 = derived from the LDS budget (see tiles_for), else a
-  // value picked by the tuner
-  int rows_x = 0;   // rows per workgroup in the x passes
-  int kb_y = 0;     // columns per workgroup in the y pass
-  int kb_z = 0;     // columns per workgroup in the z pass
+  // value picked by the tuner; columns by precision ([1]: FP32), whose passes
+  // are different ones at many shapes
+  int rows_x = 0;           // rows per workgroup in the x passes
+  int kb_y[2] = {0, 0};     // columns per workgroup in the y pass
+  int kb_z[2] = {0, 0};     // columns per workgroup in the z pass
   int lds_cap = 65536;     // device limit per workgroup
   int lds_target = 65536;  // soft budget used for the automatic tiles
   int force_generic = 0;   // 1: never use the register-resident fast path

@@ -187,8 +187,8 @@ int shape_plan_init(ShapePlan* sp, int n1, int n2, int n3, std::string* err) {
   if (const char* e = std::getenv("OFD_GENERIC")) sp->force_generic = std::atoi(e) != 0;
   if (const char* e = std::getenv("OFD_NO_PLANE")) sp->no_plane = std::atoi(e) != 0;
   if (const char* e = std::getenv("OFD_PLANE_SPLIT")) sp->plane_split = std::atoi(e);
-  if (const char* e = std::getenv("OFD_KB_Y")) sp->kb_y = std::atoi(e);
-  if (const char* e = std::getenv("OFD_KB_Z")) sp->kb_z = std::atoi(e);
+  if (const char* e = std::getenv("OFD_KB_Y")) sp->kb_y[0] = sp->kb_y[1] = std::atoi(e);
+  if (const char* e = std::getenv("OFD_KB_Z")) sp->kb_z[0] = sp->kb_z[1] = std::atoi(e);
   const size_t cb = sizeof(double2);
   if (2ull * 8 * (d.M + 1) * cb > (size_t)sp->lds_cap || 2ull * 8 * (n3 + 1) * cb > (size_t)sp->lds_cap ||
       2ull * (n2 + 1) * cb > (size_t)sp->lds_cap) {
@@ -204,9 +204,10 @@ Tiles tiles_for(const ShapePlan& sp, int nf, int cbytes) {
   const GridDims& d = sp.d;
   Tiles t;
   const long long tgt = sp.lds_target;
+  const int ky = sp.kb_y[cbytes == sizeof(float2)], kz = sp.kb_z[cbytes == sizeof(float2)];
   t.rows = sp.rows_x > 0 ? sp.rows_x : clampi(tgt / (2ll * nf * (d.M + 1) * cbytes), 1, 16);
-  t.kby = sp.kb_y > 0 ? sp.kb_y : clampi(tgt / (2ll * (d.n2 + 1) * cbytes), 1, 16);
-  t.kbz = sp.kb_z > 0 ? sp.kb_z : clampi(tgt / (2ll * nf * (d.n3 + 1) * cbytes), 1, 8);
+  t.kby = ky > 0 ? ky : clampi(tgt / (2ll * (d.n2 + 1) * cbytes), 1, 16);
+  t.kbz = kz > 0 ? kz : clampi(tgt / (2ll * nf * (d.n3 + 1) * cbytes), 1, 8);
   // never exceed the hard limit
   while (t.rows > 1 && 2ll * nf * t.rows * (d.M + 1) * cbytes > sp.lds_cap) --t.rows;
   while (t.kby > 1 && 2ll * t.kby * (d.n2 + 1) * cbytes > sp.lds_cap) --t.kby;

@@ -73,7 +73,7 @@ static YZ plan(const ShapePlan& sp, int kind) {
     g.B = b;
     g.W = g.w = 4;
     // a tuned tile only groups columns: results keep their bits
-    while (sp.kb_z > 0 && g.w > sp.kb_z) g.w /= 2;
+    while (sp.kb_z[0] > 0 && g.w > sp.kb_z[0]) g.w /= 2;
     while (g.w * std::max(a * tz, d.n3) > 256) g.w /= 2;
     g.nkt = (d.K1 + g.w - 1) / g.w;
     g.fw = kind == kWT4 || d.M >= 64 ? nf : 1;

@@ -17,7 +17,8 @@ std::map<const void*, std::string> names;
 std::string listed, failing;
 hipError_t last = hipSuccess;
 bool capturing = false;
-int lds = 163840;
+int lds = 163840, timings = 0, fastest = 0;
+std::map<std::string, unsigned> grids;   // blocks along x of a kernel's last launch
 unsigned host_flags = 0;
 const ofd::ReqDesc* desc = nullptr;   // the last uploaded or evaluated
 struct Call {
@@ -37,6 +38,13 @@ API void stub_fail(const char* kernel) { failing = kernel; }
 API void stub_capture(int on) { capturing = on != 0; }
 API void stub_lds(int bytes) { lds = bytes; }
 API void stub_clear() { listed.clear(); }
+// the k-th timing from now is half the others
+API void stub_fastest(int k) { timings = 0; fastest = k; }
+API int stub_grid(const char* kernel) {
+  for (const auto& g : grids)
+    if (g.first.find(kernel) != std::string::npos) return g.second;
+  return 0;
+}
 API const char* stub_listed() { return listed.c_str(); }
 API unsigned stub_host_flags() { return host_flags; }
 // fields of the descriptor the last evaluation pass was given
@@ -62,10 +70,11 @@ API hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* s, hipStream_
   *g = call.g; *b = call.b; *s = call.s; *st = call.st;
   return hipSuccess;
 }
-API hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t) {
+API hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void** args, size_t, hipStream_t) {
   const std::string& n = names[f];
   if (!failing.empty() && n.find(failing) != std::string::npos) return last = hipErrorLaunchFailure;
   listed += n + "\n";
+  grids[n] = grid.x;
   if (n.find("k_put_desc") != std::string::npos) {
     if (!capturing) std::memcpy(*static_cast<void**>(args[1]), args[0], sizeof(ofd::ReqDesc));
     desc = *static_cast<ofd::ReqDesc**>(args[1]);
@@ -110,4 +119,7 @@ API hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 API hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 API hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
 API hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-API hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 1.f; return hipSuccess; }
+API hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
+  *ms = ++timings == fastest ? 0.5f : 1.f;
+  return hipSuccess;
+}

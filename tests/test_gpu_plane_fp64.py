@@ -18,13 +18,13 @@ CASES = [((128, 128, 192), "wt"), ((128, 128, 192), "wt4"), ((64, 64, 256), "wt"
          ((32, 32, 192), "wt"), ((128, 128, 24), "wgc"), ((32, 32, 24), "spin"), ((32, 32, 24), "spin4")]
 
 
-def system(grid, kind):
+def system(grid, kind, **kw):
     """A skew system of its grid and kind and its electron count."""
     import profess_amd as pa
     lat = LAT * (0.24 * np.array(grid))[None, :]
     ne = 0.027 * abs(np.linalg.det(lat))
     opts = dict(kinetic=5, gamma=2.7) if kind == "wgc" else dict(alpha=0.9, beta=0.7) if kind[-1] == "4" else {}
-    s = pa.OFDSystem(lat, grid, ne, **opts)
+    s = pa.OFDSystem(lat, grid, ne, **opts, **kw)
     if kind.startswith("spin"):
         s.set_spin(2, fixed_mag=True)
     if kind == "wgc":

@@ -210,3 +210,27 @@ def test_tuner_reports_the_plane_pass(run, grid, kw):
     p = passes(s)
     assert s.autotune(reps=1)["plane"] == int("fast k_plane_fwd" in p), p
     """)
+
+
+def test_tiles_of_one_precision_stay_with_it(run):
+    """A mixed-precision system tuned at a length where FP32 takes the staged
+    passes: their z tile of one column is not the three-pass z tile of the
+    solve's FP64 evaluations."""
+    run("""
+    def fp64_tile(s):
+        try:
+            pa.ProjNormRhoMinimization(s, np.full(s.shape, 21.0 / s.vol), max_iter=1, max_line=1)
+        except calpot.OFDError:
+            pass   # no kernel runs
+        return stub.stub_grid(b"k_yz")
+    grid = (72, 72, 72)
+    before = fp64_tile(system(grid, precision=1))
+    stub.stub_fastest(2)
+    s = system(grid, precision=1)
+    r = s.autotune(reps=1)
+    assert before > 0 and (r["kb_z"], r["kb_y"]) == (1, 0), (before, r)
+    assert fp64_tile(s) == before and fp64_tile(system(grid, precision=1)) == before
+    t = system(grid)   # tuned in FP64: that tile, also in the FP64 evaluations of a mixed solve
+    stub.stub_fastest(2)
+    assert t.autotune(reps=1)["kb_z"] == 1 and fp64_tile(system(grid, precision=1)) > before
+    """)
