@@ -47,13 +47,15 @@ __global__ void __launch_bounds__(256) k_fin(const ReqDesc* __restrict__ descs, 
 }  // namespace fast
 
 // FP32: every shape of the line lengths below. FP64, of what the three-pass
-// evaluations (ofd_yz.hip, asked first) leave: the shapes of the
-// power-of-two plane passes (32 x 32, 64 x 64, 128 x 128), where two fused
-// passes beat the general form's three: Wang-Teter / fast against general
-// passes, 32^3 20.7 / 21.9 us, 64^3 34.5 / 35.3, 128^3 96 / 109. The general
-// passes take the rest, among them all other plane shapes (48^3 34.5 / 27.3,
-// 80^3 67.5 / 61.7, 96^3 65.2 / 64.0), two spin channels from 64^3 (59 / 53)
-// and WGC below 128^3 (32^3 31.1 / 30.1).
+// evaluations (ofd_yz.hip, asked first) leave: shapes of the power-of-two plane
+// passes, where two fused passes beat the general form's three. These are
+// Wang-Teter with the z lengths 192 and 256 that the three passes lack, WGC on
+// 128 x 128 planes and two spin channels on 32 x 32 (which keep their bits: the
+// three passes would be faster there, 32^3 28 us). A call, plane / general
+// passes: 32 x 32 x 192 39.8 / 41.1 us, 64 x 64 x 256 65 / 73, 128 x 128 x 192
+// 144 / 159, alpha != beta 64 x 64 x 192 76 / 81 and 128 x 128 x 256 288 / 282;
+// WGC 128 x 128 x 24 83 / 81, x 64 148 / 151, x 128 266 / 283, x 256 563 / 600;
+// left to the general passes, WGC 64^3 70 / 70, two channels 64 x 64 x 192 92 / 92.
 bool fast_path_ok(const ShapePlan& sp, int kind, int fp32) {
   if (!fast_path_ok_impl(sp, kind)) return false;
   if (fp32) return true;
@@ -61,7 +63,7 @@ bool fast_path_ok(const ShapePlan& sp, int kind, int fp32) {
   // only where the plane fits in LDS
   const int M = sp.d.M;
   if ((M != 16 && M != 32 && M != 64) || is_gp_len(sp.d.n3) || !plane_for<double>(sp)) return false;
-  return kind == kWGC8 ? M == 64 : (!is_spin_kind(kind) || M == 16);
+  return kind == kWGC8 ? M == 64 : (is_spin_kind(kind) ? M == 16 : sp.d.n3 >= 192);
 }
 
 

@@ -1668,8 +1668,8 @@ template <auto K> static inline void allow_lds(size_t lds) {
   }
 }
 
-template <typename R, int M, int KIND, int INMODE, int OUTMODE>
-static void launch_x(const ShapePlan& sp, const FastTiles& ft, const ReqDesc* dd, int nb, hipStream_t st, bool fwd,
+template <typename R, int M, int KIND, int INMODE, int OUTMODE, bool FWD>
+static void launch_x(const ShapePlan& sp, const FastTiles& ft, const ReqDesc* dd, int nb, hipStream_t st,
                      const typename V2<R>::T* tw, const typename V2<R>::T* tws) {
   using namespace fast;
   using C = typename V2<R>::T;
@@ -1681,7 +1681,7 @@ static void launch_x(const ShapePlan& sp, const FastTiles& ft, const ReqDesc* dd
     const int ntile = (int)((nrows + RPB - 1) / RPB);
     const size_t lds = (size_t)RPB * NF * GPD<M>::LINE * sizeof(C);
     const dim3 grid(ntile, nb), block(RPB * NF * GPD<M>::T);
-    if (fwd) {
+    if constexpr (FWD) {
       allow_lds<g_fx_fwd<M, KIND, INMODE, R>>(lds);
       hipLaunchKernelGGL((g_fx_fwd<M, KIND, INMODE, R>), grid, block, lds, st, dd, sp.d, tw, tws);
     } else {
@@ -1691,7 +1691,7 @@ static void launch_x(const ShapePlan& sp, const FastTiles& ft, const ReqDesc* dd
     return;
   } else {
   constexpr int T = P2<M>::R2;
-  if (fwd) {
+  if constexpr (FWD) {
     constexpr int RPB = fast::inv_rpb(NF, T);
     const long long nrows = (long long)sp.d.n2 * sp.d.n3;
     const int ntile = (int)((nrows + RPB - 1) / RPB);
@@ -1802,7 +1802,8 @@ template <int KIND> static inline bool plane_split_ok(const ShapePlan& sp) {
 // forward passes), 1 the whole plane, 2 the split form. (Four classes, a
 // quarter of the rows per workgroup, measured slower at 128^3: the plane pass
 // no faster, 26.5 us, and the z pass's radix-4 join 7.7 us dearer.)
-template <typename R, int KIND, int INMODE>
+// PM: the plane's half row length where it is known, 0: by the shape.
+template <typename R, int KIND, int INMODE, int PM = 0>
 static int try_plane(const ShapePlan& sp, const ReqDesc* dd, int nb, hipStream_t st, const typename V2<R>::T* twx,
                      const typename V2<R>::T* tws, const typename V2<R>::T* twy, int fo, int fn) {
   if (sp.no_plane) return 0;
@@ -1819,15 +1820,16 @@ static int try_plane(const ShapePlan& sp, const ReqDesc* dd, int nb, hipStream_t
     return launch_plane<R, M, N2, KIND, INMODE>(sp, dd, nb, st, twx, tws, twy, fo, fn) ? 1 : 0;
   };
   using std::integral_constant;
-  if (sp.d.M == 64 && sp.d.n2 == 128) return go(integral_constant<int, 64>(), integral_constant<int, 128>());
-  if (sp.d.M == 32 && sp.d.n2 == 64) return go(integral_constant<int, 32>(), integral_constant<int, 64>());
-  if (sp.d.M == 16 && sp.d.n2 == 32) return go(integral_constant<int, 16>(), integral_constant<int, 32>());
-  if constexpr (sizeof(R) == 8) return 0;   // the general passes take the others in FP64
-  else {
-  if (sp.d.M == 48 && sp.d.n2 == 96) return go(integral_constant<int, 48>(), integral_constant<int, 96>());
-  if (sp.d.M == 40 && sp.d.n2 == 80) return go(integral_constant<int, 40>(), integral_constant<int, 80>());
-  if (sp.d.M == 24 && sp.d.n2 == 48) return go(integral_constant<int, 24>(), integral_constant<int, 48>());
-  return 0;
+  if constexpr (PM != 0) {
+    return go(integral_constant<int, PM>(), integral_constant<int, 2 * PM>());
+  } else {
+    if (sp.d.M == 64 && sp.d.n2 == 128) return go(integral_constant<int, 64>(), integral_constant<int, 128>());
+    if (sp.d.M == 32 && sp.d.n2 == 64) return go(integral_constant<int, 32>(), integral_constant<int, 64>());
+    if (sp.d.M == 16 && sp.d.n2 == 32) return go(integral_constant<int, 16>(), integral_constant<int, 32>());
+    if (sp.d.M == 48 && sp.d.n2 == 96) return go(integral_constant<int, 48>(), integral_constant<int, 96>());
+    if (sp.d.M == 40 && sp.d.n2 == 80) return go(integral_constant<int, 40>(), integral_constant<int, 80>());
+    if (sp.d.M == 24 && sp.d.n2 == 48) return go(integral_constant<int, 24>(), integral_constant<int, 48>());
+    return 0;
   }
 }
 
@@ -1879,37 +1881,45 @@ static int fast_chain(const ShapePlan& sp, const FastTiles& ft, const ReqDesc* d
       default: launch_y<R, 256, S>(sp, ft.kby, fo, fn, dd, nb, s, twy); break;
     }
   };
-  auto zlaunch = [&](hipStream_t s, int sy, int fo, int fn) {
-    switch (sp.d.n3) {
-      case 24: launch_z<R, 24, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
-      case 32: launch_z<R, 32, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
-      case 40: launch_z<R, 40, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
-      case 48: launch_z<R, 48, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
-      case 60:
-        if constexpr (sizeof(R) == 4) launch_z<R, 60, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn);
-        break;
-      case 64: launch_z<R, 64, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
-      case 80: launch_z<R, 80, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
-      case 96: launch_z<R, 96, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
-      case 120:
-        if constexpr (sizeof(R) == 4) launch_z<R, 120, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn);
-        break;
-      case 128: launch_z<R, 128, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
-      case 192: launch_z<R, 192, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
-      default: launch_z<R, 256, KIND>(sp, ft.kbz, dd, nb, s, twz, sy, twy, fo, fn); break;
+  auto zlaunch = [&](int sy) {
+    auto z = [&](auto n) { launch_z<R, decltype(n)::value, KIND>(sp, ft.kbz, dd, nb, st, twz, sy, twy, 0, NF); };
+    using std::integral_constant;
+    // FP64 Wang-Teter comes here with the z lengths the three passes lack
+    if constexpr (sizeof(R) == 8 && (KIND == kWT3 || KIND == kWT4)) {
+      if (sp.d.n3 == 192) z(integral_constant<int, 192>());
+      else z(integral_constant<int, 256>());
+    } else {
+      switch (sp.d.n3) {
+        case 24: z(integral_constant<int, 24>()); break;
+        case 32: z(integral_constant<int, 32>()); break;
+        case 40: z(integral_constant<int, 40>()); break;
+        case 48: z(integral_constant<int, 48>()); break;
+        case 64: z(integral_constant<int, 64>()); break;
+        case 80: z(integral_constant<int, 80>()); break;
+        case 96: z(integral_constant<int, 96>()); break;
+        case 128: z(integral_constant<int, 128>()); break;
+        case 192: z(integral_constant<int, 192>()); break;
+        case 60:
+          if constexpr (sizeof(R) == 4) z(integral_constant<int, 60>());
+          break;
+        case 120:
+          if constexpr (sizeof(R) == 4) z(integral_constant<int, 120>());
+          break;
+        default: z(integral_constant<int, 256>()); break;
+      }
     }
   };
   if constexpr (sizeof(R) == 8) {
     // the plane shapes only (fast_path_ok)
-    const int pl = try_plane<R, KIND, INMODE>(sp, dd, nb, st, twx, tws, twy, 0, NF);
+    const int pl = try_plane<R, KIND, INMODE, M>(sp, dd, nb, st, twx, tws, twy, 0, NF);
     if (pl == 0) return -1;
-    zlaunch(st, pl, 0, NF);
+    zlaunch(pl);
     launch_y<R, 2 * M, +1>(sp, ft.kby, 0, NF, dd, nb, st, twy);
     if (gen_inverse(sp, 0)) gen_rows_inv(sp, KIND, INMODE, OUTMODE, dd, nb, st);
-    else if constexpr (M < 64) launch_x<R, M, KIND, INMODE, OUTMODE>(sp, ft, dd, nb, st, false, twx, tws);
+    else if constexpr (M < 64) launch_x<R, M, KIND, INMODE, OUTMODE, false>(sp, ft, dd, nb, st, twx, tws);
   } else {
     const bool plane = plane_for<R>(sp);
-    if (!plane) launch_x<R, M, KIND, INMODE, OUTMODE>(sp, ft, dd, nb, st, true, twx, tws);
+    if (!plane) launch_x<R, M, KIND, INMODE, OUTMODE, true>(sp, ft, dd, nb, st, twx, tws);
     int sy = 1;
     if (plane) {
       const int pl = try_plane<R, KIND, INMODE>(sp, dd, nb, st, twx, tws, twy, 0, NF);
@@ -1917,9 +1927,9 @@ static int fast_chain(const ShapePlan& sp, const FastTiles& ft, const ReqDesc* d
     } else {
       ylaunch(std::integral_constant<int, -1>(), st, 0, NF);
     }
-    zlaunch(st, sy, 0, NF);
+    zlaunch(sy);
     ylaunch(std::integral_constant<int, +1>(), st, 0, NF);
-    launch_x<R, M, KIND, INMODE, OUTMODE>(sp, ft, dd, nb, st, false, twx, tws);
+    launch_x<R, M, KIND, INMODE, OUTMODE, false>(sp, ft, dd, nb, st, twx, tws);
   }
   return 0;
 }
@@ -1936,11 +1946,17 @@ static int fast_eval_t(const ShapePlan& sp, const ReqDesc* dd, int nb, hipStream
   }
   (void)f32;
   int rc = 0;
-  if constexpr (sizeof(R) == 8) {   // the plane shapes
-    switch (sp.d.M) {
-      case 16: rc = fast_chain<R, KIND, INMODE, OUTMODE, 16>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-      case 32: rc = fast_chain<R, KIND, INMODE, OUTMODE, 32>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
-      default: rc = fast_chain<R, KIND, INMODE, OUTMODE, 64>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+  if constexpr (sizeof(R) == 8) {   // the plane shapes of the kind (fast_path_ok)
+    if constexpr (KIND == kWGC8) {
+      rc = fast_chain<R, KIND, INMODE, OUTMODE, 64>(sp, ft, dd, nb, st, twx, tws, twy, twz);
+    } else if constexpr (is_spin_kind(KIND)) {
+      rc = fast_chain<R, KIND, INMODE, OUTMODE, 16>(sp, ft, dd, nb, st, twx, tws, twy, twz);
+    } else {
+      switch (sp.d.M) {
+        case 16: rc = fast_chain<R, KIND, INMODE, OUTMODE, 16>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+        case 32: rc = fast_chain<R, KIND, INMODE, OUTMODE, 32>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+        default: rc = fast_chain<R, KIND, INMODE, OUTMODE, 64>(sp, ft, dd, nb, st, twx, tws, twy, twz); break;
+      }
     }
   } else {
     switch (sp.d.M) {
