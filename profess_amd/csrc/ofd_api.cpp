@@ -85,7 +85,9 @@ void stream_put(hipStream_t s) {
 // Pinned host slots of kNSum doubles, one per context, from slabs of 64 KiB
 // that stay with the process (as many as the contexts alive at once need): a
 // context then costs no hipHostMalloc or hipHostFree of its own, which wait
-// for the whole device.
+// for the whole device. Coherent, as the host reads while the kernel that
+// stores still runs (by default HIP_HOST_COHERENT decides), and portable, as a
+// slot goes to contexts of any device.
 std::mutex g_slot_mu;
 std::vector<double*> g_slots;
 constexpr size_t kSlotDoubles = 16, kSlabSlots = 512;
@@ -93,7 +95,8 @@ double* slot_get() {
   std::lock_guard<std::mutex> lk(g_slot_mu);
   if (g_slots.empty()) {
     void* p = nullptr;
-    HIPCHK(hipHostMalloc(&p, kSlabSlots * kSlotDoubles * sizeof(double), hipHostMallocDefault));
+    HIPCHK(hipHostMalloc(&p, kSlabSlots * kSlotDoubles * sizeof(double),
+                         hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent));
     for (size_t i = 0; i < kSlabSlots; ++i) g_slots.push_back(static_cast<double*>(p) + i * kSlotDoubles);
   }
   double* s = g_slots.back();

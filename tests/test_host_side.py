@@ -234,3 +234,13 @@ def test_tiles_of_one_precision_stay_with_it(run):
     stub.stub_fastest(2)
     assert t.autotune(reps=1)["kb_z"] == 1 and fp64_tile(system(grid, precision=1)) > before
     """)
+
+
+def test_polled_slots_are_coherent_and_portable(run):
+    """The host polls a slot while the kernel that stores into it runs, and the
+    slots serve the contexts of every device."""
+    run("""
+    s = system((24, 24, 24))
+    portable, coherent = 0x1, 0x40000000
+    assert stub.stub_host_flags() & (portable | coherent) == portable | coherent
+    """)
