@@ -264,11 +264,12 @@ struct Cols {
   unsigned ncol, inner, outer, es;
 };
 
-// Element access by 32-bit byte offset from a workgroup-uniform base (a
-// field's bytes stay below 2^28 at the lengths served here): scalar base and
-// one offset register per element. offs() hides an offset from the optimizer
+// Element access by 32-bit byte offset from a workgroup-uniform base (the
+// largest field served here, 512 x 256 x 256, takes 2^28 bytes and a plane):
+// scalar base and one offset register per element. offs() hides an offset from the optimizer
 // where a kernel uses it again, so that the elements' offsets are formed anew
 // (one add each) instead of staying alive through the transforms.
+static_assert((256ull + 1) * 256 * 256 * sizeof(double2) < 1ull << 32, "offsets within a field");
 __device__ __forceinline__ double2 ld16(gptr<const double2> b, unsigned off) {
   return ldc((gptr<const double2>)((gptr<const char>)b + off));
 }
@@ -428,7 +429,11 @@ __global__ void __launch_bounds__(256) k_zgop(const ReqDesc* __restrict__ descs,
 // z columns of the WGC fields with the coupled operator, as fast::k_fz_wgc:
 // blockIdx.y = 0 Hartree and vW, 1 and 2 the rho^alpha and rho^beta blocks
 // (A, B, C), which leave (c', b', a') = (K3 A, K2 A + K4 B, K1 A + K2 B +
-// K3 C) in the slots of (A, B, C).
+// K3 C) in the slots of (A, B, C). Bound by the line's three arrays in
+// registers: 170 to 252 VGPRs and two waves per SIMD from 84 points on. At 128,
+// 160, 162, 192, 224, 240, 252 and 256 points it takes 2 to 10 registers more,
+// at 200 and with radices of 21 and more 36 to 234, and runs one wave. So it
+// does at 256^3, in 755 us; the two-column form before it took 825 with two.
 template <int N>
 __global__ void __launch_bounds__(256) k_zwgc(const ReqDesc* __restrict__ descs, GridDims d,
                                               const double2* __restrict__ tw, int kb) {
@@ -545,8 +550,11 @@ constexpr int row_rpb(int m, int nf, int t, int bytes) {
 // exchange one real component at a time and run their epilogue over the two
 // halves of each row in turn (columns m < R1/2 of every thread are the row's
 // first M reals): at 16 points a thread complex lines leave 9 waves per CU
-// (256^3 WT 221 -> 200 us for the pass, 120^3 30.7 -> 28.0). With fewer points
-// a thread the complex lines are faster (180^3 58.8 against 67.5 us).
+// (256^3 WT 263 -> 244 us for the pass, 120 x 125 x 240 54.3 -> 53.8). With
+// fewer points a thread the complex lines are faster (200^3 92 against 99 us).
+// The power-of-two form that this pass replaced at 256^3 took 232 us for WT
+// with eight rows on 192 lanes (here five on 120 of 128) and 453 for WGC (here
+// 437); the call gained more before it than it lost there (1055 -> 980 us).
 template <int M> struct InvLine {
   static constexpr bool SC = L<M>::R1 % 2 == 0 && std::max(L<M>::NC, L<M>::NS) >= 15;
   static constexpr int LINE = L<M>::LINE;   // reals (SC) or complex

@@ -539,9 +539,10 @@ __global__ void __launch_bounds__(NT) k_finalize(const ReqDesc* __restrict__ des
   }
 }
 
-// 1024 threads where 256 would take three rounds or more: 256^3 WT (32768
-// partials) 986.6 -> 982.9 us a call, WGC (65536) 2613.5 -> 2606.6, 200^3 within
-// noise; up to 4096 partials (128^3: 2048) the 256 threads stay.
+// 1024 threads where 256 would take three rounds or more: 256^3 WT (13108
+// partials, five rows a workgroup) 986.6 -> 982.9 us a call, WGC (32768, two)
+// 2613.5 -> 2606.6, 200^3 within noise; up to 4096 partials (128^3: 2048) the
+// 256 threads stay.
 static int finalize_threads(int nwg) { return nwg > 4096 ? 1024 : 256; }
 
 // ============================================================ host launchers
