@@ -148,7 +148,9 @@ int ofd_calpot_device(ofd_ctx* ctx, const double* rho_device, int opt_sqrt, doub
 /* Asynchronous form for device-resident callers (no reference counterpart:
  * the reference is synchronous): enqueues the evaluation on the context's
  * stream and returns at once. sums9_device (device, 9 doubles, may be NULL)
- * receives the raw energy sums; ofd_sums_to_etable turns them into eTable. */
+ * receives the raw energy sums; ofd_sums_to_etable turns them into eTable.
+ * While the caller captures the context's stream, a call whose arguments differ
+ * from the last one's is refused (ofd_calpot_noalloc can be captured). */
 int ofd_calpot_enqueue(ofd_ctx* ctx, const double* rho_device, int opt_sqrt, double* potential_device,
                        double* sums9_device);
 int ofd_sums_to_etable(const ofd_ctx* ctx, const double* sums9, double* etable9);
